@@ -83,6 +83,17 @@ struct View {
 };
 View dense_view(void* p, const Shape& sh, int es = 8);
 
+// stages of an FFT of length M with factors 2, 3, 5, 7 only (smooth_fft.hpp): radix rad[s] = M / mp[s]
+// after span span[s]; r*: the same radices in reverse order (the inverse transform of a fused pass, which
+// starts where the forward one ends)
+constexpr int kSmoothStages = 5;
+struct SmoothPlan {
+    int M = 0, nst = 0, T = 0;             // T: threads per pencil, the largest M / rad[s]
+    int rad[kSmoothStages] = {0}, mp[kSmoothStages] = {0}, span[kSmoothStages] = {0}, inv[kSmoothStages] = {0}, stride[kSmoothStages] = {0};
+    int rspan[kSmoothStages] = {0}, rinv[kSmoothStages] = {0}, rstride[kSmoothStages] = {0};
+};
+bool smooth_plan(int M, SmoothPlan& p);   // smooth.hip; false when M has another prime factor or is out of range
+
 // everything one launch of the generic pencil kernel needs (one component)
 struct PassDesc {
     int d = 0;
@@ -105,10 +116,25 @@ struct PassDesc {
     int na = 1;             // extent along fa
     int alias = 0;          // 1: the second FFT buffer reuses the pencil buffer
     int fastk = 0;          // fast kernels of rowpass.hip instead of the generic one: 1 row r2r, 2 paired real columns,
-                            // 3 row r2c / c2r, 4 column r2r, 5 column c2c, 6 row c2c
+                            // 3 row r2c / c2r, 4 column r2r, 5 column c2c, 6 row c2c; with sm.M > 0 the same shapes
+                            // on the kernels of smooth.hip (2: strided r2c / c2r)
     int vec = 0;            // fast kernels: pencils start 16-byte aligned in source and destination
     int nt = 0;             // row r2r kernel: its vector accesses are non-temporal (both arrays 128 MiB or more)
     const double* aux = nullptr;   // fast kernels: pre / post twiddle table
+    SmoothPlan sm;          // M > 0: kernels of smooth.hip, their stages (sm.T threads per pencil, ppb pencils per block)
+};
+
+// the last direction of the general path, c2c of a smooth length, with the multiply (smooth.hip)
+struct SmoothZArgs {
+    void* d = nullptr;           // field before the transform, in place: complex, x fastest, rows s_col apart
+    const void* g = nullptr;     // normfact G, [y'][tile][kz'][tx]
+    const double* tw = nullptr;  // M-point twiddle table
+    int nx = 1, nother = 1, nin = 1, tx = 8;
+    int mirror = 0;              // 1: the rows y and nother - y share their G
+    int f32 = 0;                 // data and G stored as float (FP64 arithmetic)
+    int lda = 1;
+    long long s_col = 1, s_other = 1, comp = 0;
+    SmoothPlan sm;
 };
 
 // the last direction of the general path as one r2c -> normfact G -> c2r launch (rowpass.hip):

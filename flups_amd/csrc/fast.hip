@@ -1269,6 +1269,8 @@ void launch_col_rz(const RzArgs& A, hipStream_t s);   // rowpass.hip
 void launch_row_rz(const RzArgs& A, hipStream_t s);
 bool row_rz_len_ok(int M);
 bool split_pq(int n, int& pf, int& q);
+int smooth_z_tile(int M);                              // smooth.hip
+void launch_smooth_z(const SmoothZArgs& A, hipStream_t s);
 
 struct HybridZ {
     int M = 0, nx = 0, ny = 0, nz = 0, lda = 1, gtx = 8;
@@ -1278,7 +1280,8 @@ struct HybridZ {
     double normfact = 1;
     const void* g = nullptr;     // real: the solver's spectral Green's function (not owned)
     bool f32 = false;            // FP32 stage arrays and Green's function (FP64 arithmetic)
-    int pf = 1;              // M = pf 2^k: 1, or 3 (mixed-radix column FFT, 8 pf values per thread)
+    int pf = 1;              // M = pf 2^k: 1, or 3 (mixed-radix column FFT, 8 pf values per thread), 5, 7 (thread
+                             // teams); 0: any other smooth length (smooth_z)
     bool pair = false, twod = false;
     void* green = nullptr;   // normfact * Re G, [y'][tile][kz'][gtx]
     void* tw = nullptr;      // (M / pf)-point table
@@ -1371,7 +1374,8 @@ HybridZ* make_hybrid_z(SolverImpl& s) {
     const int M = f.n_in[0];
     const bool p2 = pow2_in(M, 32, nd == 2 ? 2048 : 1024), p3 = M % 3 == 0 && pow2_in(M / 3, 8, 128),
                p5 = M % 5 == 0 && pow2_in(M / 5, 8, 128), p7 = M % 7 == 0 && pow2_in(M / 7, 8, 128);
-    if (!(p2 || p3 || p5 || p7) || sp.n[nd - 1] != M) return nullptr;
+    const int smooth_tx = p2 || p3 || p5 || p7 ? 0 : smooth_z_tile(M);
+    if (!(p2 || p3 || p5 || p7 || smooth_tx) || sp.n[nd - 1] != M) return nullptr;
     const int ny = nd == 3 ? in.n[1] : 1;
     if ((double)(M / 8) * in.n[0] * ny * 16.0 >= 4294967296.0) return nullptr;
     auto* h = new HybridZ;
@@ -1388,7 +1392,8 @@ HybridZ* make_hybrid_z(SolverImpl& s) {
     // half-width x tiles in 3-D; two columns per block in 2-D (few columns, cache-resident field)
     h->gtx = nd == 2 ? 2 : 4;
     h->twod = nd == 2;
-    h->pf = p2 ? 1 : p3 ? 3 : p5 ? 5 : 7;
+    h->pf = p2 ? 1 : p3 ? 3 : p5 ? 5 : p7 ? 7 : 0;
+    if (h->pf == 0) h->gtx = smooth_tx;
     if (h->pf >= 5) {   // thread teams, one row per block: no mirror pairing, tiles by length (LDS M gtx complex:
                         // 48 KB up to M = 384, then 4 columns: 28 / 40 / 56 KB at M = 448 / 640 / 896)
         h->pair = false;
@@ -1406,7 +1411,7 @@ HybridZ* make_hybrid_z(SolverImpl& s) {
         hipLaunchKernelGGL(compress_green, dim3(4096), dim3(256), 0, s.stream_, s.dgreen_, f32 ? nullptr : (double*)h->green,
                            f32 ? (float*)h->green : nullptr, h->nx, h->ny, M, gy, gz, h->gtx, ntx, s.normfact_);
         HIP_CHECK(hipGetLastError());
-        const auto t = twiddle_table(M / h->pf);
+        const auto t = twiddle_table(h->pf ? M / h->pf : M);
         HIP_CHECK(hipMalloc(&h->tw, t.size() * sizeof(double)));
         HIP_CHECK(hipMemcpy(h->tw, t.data(), t.size() * sizeof(double), hipMemcpyHostToDevice));
         h->dev_bytes += t.size() * sizeof(double);
@@ -1532,6 +1537,25 @@ void hybrid_z_t(const HybridZ* h, void* data, hipStream_t st) {
         A.comp = (long long)h->nx * h->ny * h->nz;
         A.normfact = h->normfact;
         launch_col_rz(A, st);
+        return;
+    }
+    if (h->pf == 0) {
+        SmoothZArgs A;
+        A.f32 = std::is_same<S, float>::value;
+        A.d = data;
+        A.g = h->green;
+        A.tw = static_cast<const double*>(h->tw);
+        A.nx = h->nx;
+        A.nother = h->ny;
+        A.nin = h->nz;
+        A.tx = h->gtx;
+        A.mirror = h->pair;
+        A.lda = h->lda;
+        A.s_col = (long long)h->nx * h->ny;
+        A.s_other = h->nx;
+        A.comp = (long long)h->nx * h->ny * h->nz;
+        smooth_plan(h->M, A.sm);
+        launch_smooth_z(A, st);
         return;
     }
     ColArgs z{};

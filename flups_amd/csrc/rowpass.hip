@@ -48,6 +48,11 @@ bool fft_len_ok(int n, int lo, int hi, int maxpf) {
     if (pf == 1) return q >= lo && q <= hi;
     return pf <= maxpf && q >= 8 && q <= 128;
 }
+// the lengths of the kernels of smooth.hip (smooth = true) take the same shapes of passes
+bool len_ok(bool smooth, int n, int lo, int hi, int maxpf) {
+    SmoothPlan p;
+    return smooth ? smooth_plan(n, p) : fft_len_ok(n, lo, hi, maxpf);
+}
 }  // namespace
 
 namespace {
@@ -63,13 +68,13 @@ bool c2c_pencil_ok(const PassDesc& P) {
 
 namespace {
 // the plan semantics the r2r pencil kernels reproduce (kinds, length, offsets, corrections)
-bool r2r_plan_fits(const PassDesc& P) {
+bool r2r_plan_fits(const PassDesc& P, bool smooth) {
     const int k = P.kind;
     const int n = P.n, h = r2r_h(k, n);
     if (P.op != OP_R2R) return false;
     const bool e00 = k == REDFT00 || k == RODFT00;
     if (!(e00 || k == REDFT10 || k == REDFT01 || k == REDFT11 || k == RODFT10 || k == RODFT01 || k == RODFT11)) return false;
-    if ((!e00 && n % 2) || !fft_len_ok(h, 16, 1024, 7)) return false;
+    if ((!e00 && n % 2) || !len_ok(smooth, h, 16, 1024, 7)) return false;
     if (!(P.src_nf == 1 && P.dst_nf == 1 && P.nf_in == 1 && P.nf_out == 1 && P.r2r_stride == 1 && P.pen_in == P.pen_out &&
           P.pen_in >= n && P.pen_in <= n + 2 && P.gshift >= 0 && P.sshift >= 0))
         return false;
@@ -84,10 +89,10 @@ bool r2r_plan_fits(const PassDesc& P) {
 }
 }  // namespace
 
-bool row_r2r_fits(const PassDesc& P) { return r2r_plan_fits(P) && P.src_s[P.d] == 1 && P.dst_s[P.d] == 1; }
+bool row_r2r_fits(const PassDesc& P, bool smooth) { return r2r_plan_fits(P, smooth) && P.src_s[P.d] == 1 && P.dst_s[P.d] == 1; }
 
-bool col_r2r_fits(const PassDesc& P) {
-    return r2r_plan_fits(P) && P.fa != P.d && P.src_s[P.fa] == 1 && P.dst_s[P.fa] == 1 && (P.n1 * P.n2) % P.na == 0;
+bool col_r2r_fits(const PassDesc& P, bool smooth) {
+    return r2r_plan_fits(P, smooth) && P.fa != P.d && P.src_s[P.fa] == 1 && P.dst_s[P.fa] == 1 && (P.n1 * P.n2) % P.na == 0;
 }
 
 // pre / post twiddles of the row r2r kernels, (H + 1) complex each, exact to rounding
@@ -120,19 +125,34 @@ std::vector<double> row_r2r_table(int kind, int n) {
     return t;
 }
 
-bool row_rc_fits(const PassDesc& P) {
+namespace {
+// the plan semantics of the packed r2c / c2r pencils (either layout)
+bool rc_plan_fits(const PassDesc& P) {
     const int n = P.n, h = n / 2;
-    if (!(P.op == OP_R2C || P.op == OP_C2R) || n % 2 || !fft_len_ok(h, 16, 1024, 7)) return false;
+    if (!(P.op == OP_R2C || P.op == OP_C2R) || n % 2) return false;
     const bool fwd = P.op == OP_R2C;
-    const int d = P.d;
-    if (P.src_s[d] != 1 || P.dst_s[d] != 1 || P.si != 0 || P.so != 0 || (P.post & ~POST_PERIOD) || P.gshift < 0 || P.sshift < 0)
+    if (P.si != 0 || P.so != 0 || (P.post & ~POST_PERIOD) || P.gshift < 0 || P.sshift < 0)
         return false;
     // the periodic copy lands inside the pencil (r2c: complex value n_out - 1, c2r: real value n)
     if ((P.post & POST_PERIOD) && (fwd ? P.n_out_plan - 1 >= P.pen_out || P.n_out_plan < 1 : n >= P.pen_out)) return false;
-    // buffer of the pencil in LDS: at most 2H + H/4 doubles
-    if (P.pen_in * P.nf_in > 2 * h + h / 4 || P.pen_out * P.nf_out > 2 * h + h / 4) return false;
     if (fwd) return P.nf_in == 1 && P.src_nf == 1 && P.nf_out == 2 && P.dst_nf == 2 && P.pen_in >= n && P.pen_out >= h + 1;
     return P.nf_in == 2 && P.src_nf == 2 && P.nf_out == 1 && P.dst_nf == 1 && P.pen_in >= h + 1 && P.pen_out >= n;
+}
+}  // namespace
+
+bool row_rc_fits(const PassDesc& P, bool smooth) {
+    const int h = P.n / 2;
+    if (!rc_plan_fits(P) || P.src_s[P.d] != 1 || P.dst_s[P.d] != 1 || !len_ok(smooth, h, 16, 1024, 7)) return false;
+    // buffer of the pencil in LDS: at most 2H + H/4 doubles (the kernels of smooth.hip size it at the launch)
+    return smooth || (P.pen_in * P.nf_in <= 2 * h + h / 4 && P.pen_out * P.nf_out <= 2 * h + h / 4);
+}
+
+// strided r2c / c2r of a smooth length, neighbouring pencils along a unit-stride dimension
+bool col_rc_fits(const PassDesc& P) {
+    SmoothPlan p;
+    const int fa = P.fa;
+    return rc_plan_fits(P) && fa != P.d && P.src_s[fa] == 1 && P.dst_s[fa] == 1 && (P.n1 * P.n2) % P.na == 0 &&
+           smooth_plan(P.n / 2, p);
 }
 
 bool col_real_fits(const PassDesc& P) {
@@ -158,18 +178,18 @@ bool col_real_fits(const PassDesc& P) {
     return P.si == 0 && P.so == 0 && P.gshift == 0 && P.sshift == 0 && (P.n1 * P.n2) % P.na == 0;
 }
 
-bool col_c2c_fits(const PassDesc& P) {
+bool col_c2c_fits(const PassDesc& P, bool smooth) {
     const int n = P.n;
-    if (P.op != OP_C2C || !fft_len_ok(n, 32, 2048, 7) || P.M != n) return false;
+    if (P.op != OP_C2C || !len_ok(smooth, n, 32, 2048, 7) || P.M != n) return false;
     const int d = P.d, fa = P.fa;
     if (fa == d || P.src_s[fa] != 1 || P.dst_s[fa] != 1 || (P.n1 * P.n2) % P.na != 0) return false;
     if (!(P.nf_in == 2 && P.nf_out == 2 && P.src_nf == 2 && P.dst_nf == 2 && c2c_pencil_ok(P))) return false;
     return P.si == 0 && P.so == 0 && P.gshift >= 0 && P.sshift >= 0 && P.src_nd >= 1 && P.dst_nd >= 1;
 }
 
-bool row_c2c_fits(const PassDesc& P) {
+bool row_c2c_fits(const PassDesc& P, bool smooth) {
     const int n = P.n, d = P.d;
-    if (P.op != OP_C2C || !fft_len_ok(n, 16, 1024, 7) || P.M != n) return false;
+    if (P.op != OP_C2C || !len_ok(smooth, n, 16, 1024, 7) || P.M != n) return false;
     if (P.src_s[d] != 1 || P.dst_s[d] != 1) return false;
     if (!(P.nf_in == 2 && P.nf_out == 2 && P.src_nf == 2 && P.dst_nf == 2 && c2c_pencil_ok(P))) return false;
     return P.si == 0 && P.so == 0 && P.gshift >= 0 && P.sshift >= 0 && P.src_nd >= 1 && P.dst_nd >= 1;

@@ -25,21 +25,26 @@ namespace flups {
 size_t generic_lds_bytes(const PassDesc& P, int ppb);
 bool generic_alias(const PassDesc& P);
 void launch_generic(const PassDesc& P, hipStream_t s);
-bool row_r2r_fits(const PassDesc& P);
+bool row_r2r_fits(const PassDesc& P, bool smooth = false);
 bool col_real_fits(const PassDesc& P);
 void launch_col_real(const PassDesc& P, hipStream_t s);
-bool row_rc_fits(const PassDesc& P);
+bool row_rc_fits(const PassDesc& P, bool smooth = false);
+bool col_rc_fits(const PassDesc& P);
 void launch_row_rc(const PassDesc& P, hipStream_t s);
 std::vector<double> row_r2r_table(int kind, int n);
 void launch_row_r2r(const PassDesc& P, hipStream_t s);
-bool col_r2r_fits(const PassDesc& P);
-bool col_c2c_fits(const PassDesc& P);
+bool col_r2r_fits(const PassDesc& P, bool smooth = false);
+bool col_c2c_fits(const PassDesc& P, bool smooth = false);
 bool split_pq(int n, int& pf, int& q);
 int r2r_h(int kind, int n);
-bool row_c2c_fits(const PassDesc& P);
+bool row_c2c_fits(const PassDesc& P, bool smooth = false);
 void launch_row_c2c(const PassDesc& P, hipStream_t s);
 void launch_col_c2c(const PassDesc& P, hipStream_t s);
 void launch_col_r2r(const PassDesc& P, hipStream_t s);
+bool smooth_col_tile(PassDesc& P, int n);   // smooth.hip
+void launch_smooth_col(const PassDesc& P, hipStream_t s);
+bool smooth_pen_tile(PassDesc& P, int h, bool col);
+void launch_smooth_pen(const PassDesc& P, bool col, hipStream_t s);
 FastPlan* make_fast_plan(SolverImpl& s);   // nullptr if the fused pipeline does not apply
 void destroy_fast_plan(FastPlan* f);
 void fast_solve(FastPlan* f, double* field, const double* rhs, const View& uin, const View& uout, hipStream_t s,
@@ -462,6 +467,8 @@ PassDesc SolverImpl::pass_desc(const DirPlan& p, int comp, bool forward, const V
         P.vec = ((uintptr_t)real % (2 * res) == 0) && rs[P.d] % 2 == 0 && rs[P.fb] % 2 == 0 && P.na % 2 == 0;
         return P;
     }
+    // the same shapes at the other lengths with factors 2, 3, 5, 7: run-time mixed radix
+    if (!std::getenv("FLUPS_GENERIC_PASS") && smooth_pass(P)) return P;
     P.alias = generic_alias(P) ? 1 : 0;
     const size_t per_pen = generic_lds_bytes(P, 1);
     FLUPS_REQUIRE(per_pen <= lds_budget_, "pencil of %d elements (transform length %d) does not fit the general path's LDS",
@@ -476,7 +483,32 @@ PassDesc SolverImpl::pass_desc(const DirPlan& p, int comp, bool forward, const V
     return P;
 }
 
+// a pass for the kernels of smooth.hip (sm.M > 0): its shape's code, tile and tables (false: none fits)
+bool SolverImpl::smooth_pass(PassDesc& P) {
+    PassDesc Q = P;
+    const bool row = row_r2r_fits(P, true) || row_rc_fits(P, true) || row_c2c_fits(P, true);
+    if (row || col_r2r_fits(P, true) || col_rc_fits(P)) {
+        const int h = P.op == OP_R2R ? r2r_h(P.kind, P.n) : P.op == OP_C2C ? P.n : P.n / 2;
+        if (!smooth_pen_tile(Q, h, !row)) return false;
+        P = Q;
+        P.fastk = P.op == OP_R2R ? (row ? 1 : 4) : P.op == OP_C2C ? 6 : (row ? 3 : 2);
+        P.tw = twiddles(h);
+        P.aux = P.op == OP_R2R ? r2r_table(P.kind, P.n) : twiddles(P.n);
+        return true;
+    }
+    if (!col_c2c_fits(P, true) || !smooth_col_tile(Q, P.n)) return false;
+    P = Q;
+    P.fastk = 5;
+    P.tw = twiddles(P.n);
+    return true;
+}
+
 void SolverImpl::run_pass(PassDesc P) {
+    if (P.sm.M > 0) {
+        if (P.fastk == 5) launch_smooth_col(P, stream_);
+        else launch_smooth_pen(P, P.fastk == 2 || P.fastk == 4, stream_);
+        return;
+    }
     if (P.fastk == 1) launch_row_r2r(P, stream_);
     else if (P.fastk == 2) launch_col_real(P, stream_);
     else if (P.fastk == 3) launch_row_rc(P, stream_);

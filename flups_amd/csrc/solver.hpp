@@ -110,6 +110,7 @@ class SolverImpl {
     void plan_fft(PassDesc& P, int M);
     PassDesc pass_desc(const DirPlan& p, int comp, bool forward, const View& src, const View& dst, const Shape& tin,
                        const Shape& tout, int gshift, int sshift);
+    bool smooth_pass(PassDesc& P);
     void run_pass(PassDesc P);
     void fill_green_args(GreenArgs& A, const double hfact[3], const double kfact[3], const double koffset[3],
                          const double symstart[3], double length, int nunb);
