@@ -89,6 +89,7 @@ View dense_view(void* p, const Shape& sh, int es = 8);
 constexpr int kSmoothStages = 5;
 struct SmoothPlan {
     int M = 0, nst = 0, T = 0;             // T: threads per pencil, the largest M / rad[s]
+    int wide = 0;                          // 1: a radix above 10
     int rad[kSmoothStages] = {0}, mp[kSmoothStages] = {0}, span[kSmoothStages] = {0}, inv[kSmoothStages] = {0}, stride[kSmoothStages] = {0};
     int rspan[kSmoothStages] = {0}, rinv[kSmoothStages] = {0}, rstride[kSmoothStages] = {0};
 };

@@ -1269,7 +1269,7 @@ void launch_col_rz(const RzArgs& A, hipStream_t s);   // rowpass.hip
 void launch_row_rz(const RzArgs& A, hipStream_t s);
 bool row_rz_len_ok(int M);
 bool split_pq(int n, int& pf, int& q);
-int smooth_z_tile(int M);                              // smooth.hip
+int smooth_z_tile(int M, bool f32);                          // smooth.hip
 void launch_smooth_z(const SmoothZArgs& A, hipStream_t s);
 
 struct HybridZ {
@@ -1374,7 +1374,7 @@ HybridZ* make_hybrid_z(SolverImpl& s) {
     const int M = f.n_in[0];
     const bool p2 = pow2_in(M, 32, nd == 2 ? 2048 : 1024), p3 = M % 3 == 0 && pow2_in(M / 3, 8, 128),
                p5 = M % 5 == 0 && pow2_in(M / 5, 8, 128), p7 = M % 7 == 0 && pow2_in(M / 7, 8, 128);
-    const int smooth_tx = p2 || p3 || p5 || p7 ? 0 : smooth_z_tile(M);
+    const int smooth_tx = p2 || p3 || p5 || p7 ? 0 : smooth_z_tile(M, f32);
     if (!(p2 || p3 || p5 || p7 || smooth_tx) || sp.n[nd - 1] != M) return nullptr;
     const int ny = nd == 3 ? in.n[1] : 1;
     if ((double)(M / 8) * in.n[0] * ny * 16.0 >= 4294967296.0) return nullptr;

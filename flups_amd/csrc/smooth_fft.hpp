@@ -196,21 +196,22 @@ __device__ __forceinline__ void smooth_stage(int t, int mp, int span, int inv, i
     __syncthreads();
 }
 
-#define FLUPS_SMOOTH_RADIX(R_, CALL)                                              \
-    switch (R_) {                                                                 \
-        case 2: { CALL(2); } break;                                               \
-        case 3: { CALL(3); } break;                                               \
-        case 4: { CALL(4); } break;                                               \
-        case 5: { CALL(5); } break;                                               \
-        case 6: { CALL(6); } break;                                               \
-        case 7: { CALL(7); } break;                                               \
-        case 8: { CALL(8); } break;                                               \
-        case 9: { CALL(9); } break;                                               \
-        case 10: { CALL(10); } break;                                             \
-        case 12: { CALL(12); } break;                                             \
-        case 14: { CALL(14); } break;                                             \
-        case 15: { CALL(15); } break;                                             \
-        default: { CALL(16); } break;                                             \
+// one case per radix; WIDE kernels have all of them, the others those up to 10
+#define FLUPS_SMOOTH_RADIX(R_, CALL)                                  \
+    switch (R_) {                                                     \
+        case 2: { CALL(2); } break;                                   \
+        case 3: { CALL(3); } break;                                   \
+        case 4: { CALL(4); } break;                                   \
+        case 5: { CALL(5); } break;                                   \
+        case 6: { CALL(6); } break;                                   \
+        case 7: { CALL(7); } break;                                   \
+        case 8: { CALL(8); } break;                                   \
+        case 9: { CALL(9); } break;                                   \
+        case 10: { CALL(10); } break;                                 \
+        case 12: { if constexpr (WIDE) { CALL(12); } } break;         \
+        case 14: { if constexpr (WIDE) { CALL(14); } } break;         \
+        case 15: { if constexpr (WIDE) { CALL(15); } } break;         \
+        default: { if constexpr (WIDE) { CALL(16); } } break;         \
     }
 
 }  // namespace flups
