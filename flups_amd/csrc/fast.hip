@@ -38,11 +38,15 @@
 #include <type_traits>
 #include <vector>
 
+#include "fast_args.hpp"
 #include "fft_core.hpp"
 #include "group.hpp"
 #include "solver.hpp"
 
 namespace flups {
+
+template <typename R>
+void launch_z_rot(int M, const ColArgs& a, const RotK& rk, hipStream_t st);   // zrot.hip
 
 namespace {
 
@@ -69,34 +73,6 @@ __device__ __forceinline__ void st_nt(C2<float>* p, C2<float> v) {
     __builtin_nontemporal_store(f2nt{v.x, v.y}, reinterpret_cast<f2nt*>(p));
 }
 
-// ---------------------------------------------------------------------------
-// column passes along y or z of the stage arrays
-struct ColArgs {
-    const void* src;
-    void* dst;
-    const void* green;   // z_fused only: normfact * G, [kz'][ky'][kx], kx padded to ldx
-    const void* tw;
-    int nx;              // valid x columns
-    int ldx;             // x row length in complex elements (multiple of 8/16)
-    long long s_col;     // element stride between rows of a column (src and dst share it for z; y differs below)
-    long long s_col_dst;
-    long long s_other_src, s_other_dst;   // stride of the other (batch) dimension
-    int nother;
-    int nin, nout;       // valid input rows, rows to store
-    int gy, gmy, gmz;    // z_fused: ky' extent, M1 (for ky' = min(y, M1-y)), M2
-    int cstride_src, cstride_dst;   // component strides in complex elements (low 32 bits)
-    long long comp_src, comp_dst;
-    int rev;             // 1: blocks walk the batch from its last entry
-    int xcd;             // z_fused: 1 = XCD-grouped block numbering
-    int nopair;          // z_fused: 1 = the other dim has no mirror rows (one row per block, G stored per row)
-    int x0;              // z_fused / z_rot: spectral x index of column 0 (slab offset, a multiple of TX)
-    int gntx;            // z_fused / z_rot: x tiles of one ky' row of the compressed G
-    int gtx;             // z_rot: tile width of the compressed G (a multiple of the kernel's TX)
-    const void* twm;     // z_fused with PF > 1: M-point twiddle table (tw is then the M/PF-point one)
-    int crot;            // col_fft: 1 = component c is read from slot (c + 1) mod 3 (after z_rot)
-    int nt;              // col_fft forward: 1 = non-temporal stores
-};
-
 // TX columns per block, M/8 threads per column; block = TX * M/8 threads.
 // HALF: zero-padded input of M/2 rows (forward) or output truncated to M/2 rows
 // (inverse); nin / nout are then not consulted. Lanes past nx load a valid
@@ -117,8 +93,7 @@ struct col_fft {
         const int other = blk / ntx;
         const int x = tile * TX + c;
         const bool live = x < a.nx;
-        const int cin = a.crot ? (bk.y + 1) % 3 : bk.y;   // source slot of this component
-        const C2<R>* src = reinterpret_cast<const C2<R>*>(a.src) + cin * a.comp_src + other * a.s_other_src + min(x, a.nx - 1);
+        const C2<R>* src = reinterpret_cast<const C2<R>*>(a.src) + bk.y * a.comp_src + other * a.s_other_src + min(x, a.nx - 1);
         C2<R>* dst = reinterpret_cast<C2<R>*>(a.dst) + bk.y * a.comp_dst + other * a.s_other_dst + x;
         const C2<R>* tw = reinterpret_cast<const C2<R>*>(a.tw);
         constexpr bool HIN = HALF && FWD, HOUT = HALF && !FWD;
@@ -317,19 +292,6 @@ struct z_team {
     }
 };
 
-// Rotational (Biot-Savart) z pass, in place on the three components of S1:
-// forward FFT of omega_x, omega_y, omega_z along z, psi = normfact G omega, then
-// u = curl psi = i K x psi with the derivative symbol K of each direction (the
-// wave number itself, or the symbol of the 2nd/4th/6th-order centred
-// difference), inverse FFTs, keep the first nin rows. The same y-row pairing
-// and Green's slice as z_fused. src/dothemagic_rot.ipp:102-349.
-struct RotK {
-    double kfact[3], h[3], symstart[3];
-    int order;          // 1 spectral, 2 / 4 / 6 centred differences
-    const void* sym;    // derivative symbols by mode index: x (nx), then y (M1), then z (M2), type R
-    int off[3];         // start of each direction's table
-};
-
 // derivative symbol of mode idx along d: symmetrised index (mirrored half negative),
 // k = is * kfact, then k itself (spectral) or the symbol of the 2nd/4th/6th-order
 // centred difference (src/dothemagic_rot.ipp:14-101); tabulated on the host
@@ -348,219 +310,6 @@ double rot_symbol(const RotK& k, int d, int idx) {
         default: return kk;
     }
 }
-
-// FP64: the three components' sets of NV values live together (all loads issued before the
-// first transform); in place, u_c back in slot c
-template <typename R, int M, int TX>
-__device__ __forceinline__ void z_rot_body3(const ColArgs& a, const RotK& rk, C2<R>* lds, Blk bk) {
-    constexpr int NV = 8, T = M / NV;
-    const int c = threadIdx.x % TX;
-    const int j = threadIdx.x / TX;
-    const int ntx = (a.nx + TX - 1) / TX;
-    const int blk = a.xcd ? xcd_group(bk.x, bk.nx) : bk.x;
-    const int tile = blk % ntx;
-    const int y0 = blk / ntx;
-    const int y1 = a.gmy - y0;
-    const bool pair = y0 != 0 && y1 != y0;
-    const int x = tile * TX + c;
-    const bool live = x < a.nx;
-    char* base = reinterpret_cast<char*>(a.dst) + (size_t)sizeof(C2<R>) * ((long long)tile * TX);
-    const size_t cstride = (size_t)sizeof(C2<R>) * a.comp_src;
-    const size_t rstride = (size_t)sizeof(C2<R>) * T * a.s_col;
-    const unsigned voff = (unsigned)(sizeof(C2<R>) * ((size_t)j * a.s_col + c));
-    // lanes past nx load the last valid column and store nothing
-    const unsigned loff = (unsigned)(sizeof(C2<R>) * ((size_t)j * a.s_col + min(c, a.nx - 1 - tile * TX)));
-    // the block's TX columns lie in one tile of the G layout (gtx a multiple of TX)
-    const int xg = a.x0 + tile * TX;
-    const int cg = xg % a.gtx + c;
-    const char* g = reinterpret_cast<const char*>(a.green) +
-                    sizeof(R) * ((long long)y0 * a.gntx + xg / a.gtx) * (M / 2 + 1) * a.gtx;
-    const C2<R>* tw = reinterpret_cast<const C2<R>*>(a.tw);
-    const R* sym = reinterpret_cast<const R*>(rk.sym);
-    const R kx = sym[rk.off[0] + a.x0 + min(x, a.nx - 1)];
-    for (int s = 0; s < 2; ++s) {
-        const int y = s == 0 ? y0 : y1;
-        char* b = base + (size_t)sizeof(C2<R>) * ((long long)y * a.s_other_src);
-        const R ky = sym[rk.off[1] + y];
-        C2<R> v[3][NV];
-        // the three components' loads all issued before the first FFT (its barriers would
-        // otherwise hold each component's loads back until the previous transform is done)
-#pragma unroll
-        for (int cc = 0; cc < 3; ++cc)
-#pragma unroll
-            for (int i = 0; i < NV; ++i) {
-                const int row = j + i * T;
-                v[cc][i] = row < a.nin ? *reinterpret_cast<const C2<R>*>(b + cc * cstride + i * rstride + loff) : C2<R>{0, 0};
-            }
-#pragma unroll
-        for (int cc = 0; cc < 3; ++cc) {
-            column_fft<R, M, true, TX>(v[cc], lds + c, j, tw);
-        }
-        // G of this tile, loaded after the forward transforms (fewer registers live during them)
-        R gv[NV];
-#pragma unroll
-        for (int i = 0; i < NV; ++i) {
-            const int kz = j + i * T;
-            gv[i] = *reinterpret_cast<const R*>(g + (unsigned)(sizeof(R) * (min(kz, M - kz) * a.gtx + cg)));
-        }
-#pragma unroll
-        for (int i = 0; i < NV; ++i) {
-            const R kz = sym[rk.off[2] + j + i * T];
-            const C2<R> wx = {v[0][i].x * gv[i], v[0][i].y * gv[i]};
-            const C2<R> wy = {v[1][i].x * gv[i], v[1][i].y * gv[i]};
-            const C2<R> wz = {v[2][i].x * gv[i], v[2][i].y * gv[i]};
-            // u = i K x w: (K x w) then multiply by i: (p + i q) i = -q + i p
-            const C2<R> cx = {ky * wz.x - kz * wy.x, ky * wz.y - kz * wy.y};
-            const C2<R> cy = {kz * wx.x - kx * wz.x, kz * wx.y - kx * wz.y};
-            const C2<R> cz = {kx * wy.x - ky * wx.x, kx * wy.y - ky * wx.y};
-            v[0][i] = {-cx.y, cx.x};
-            v[1][i] = {-cy.y, cy.x};
-            v[2][i] = {-cz.y, cz.x};
-        }
-#pragma unroll
-        for (int cc = 0; cc < 3; ++cc) {
-            column_fft<R, M, false, TX>(v[cc], lds + c, j, tw);
-            if (live) {
-#pragma unroll
-                for (int i = 0; i < NV; ++i) {
-                    const int row = j + i * T;
-                    if (row < a.nout) *reinterpret_cast<C2<R>*>(b + cc * cstride + i * rstride + voff) = v[cc][i];
-                }
-            }
-        }
-        if (!pair) break;   // uniform over the block
-    }
-}
-
-// FP32: two sets of NV values live at a time (see the comment inside); u_c lands in slot
-// (c + 1) mod 3, and the inverse y pass reads it there (ColArgs::crot). For FP64 this order
-// (one component read and transformed twice) is slower than the three-set one: 32.5 against
-// 27.6 ms at 513^3 x 3, the fewer registers still leave one block of 512 threads per CU; FP32:
-// 17.6 against 18.7 ms (no spills at 128 registers, where the three-set order spilled 20)
-template <typename R, int M, int TX>
-__device__ __forceinline__ void z_rot_body2(const ColArgs& a, const RotK& rk, C2<R>* lds, C2<R>* ltw, Blk bk) {
-    constexpr int NV = 8, T = M / NV;
-    const int c = threadIdx.x % TX;
-    const int j = threadIdx.x / TX;
-    const int ntx = (a.nx + TX - 1) / TX;
-    const int blk = a.xcd ? xcd_group(bk.x, bk.nx) : bk.x;
-    const int tile = blk % ntx;
-    const int y0 = blk / ntx;
-    const int y1 = a.gmy - y0;
-    const bool pair = y0 != 0 && y1 != y0;
-    const int x = tile * TX + c;
-    const bool live = x < a.nx;
-    char* base = reinterpret_cast<char*>(a.dst) + (size_t)sizeof(C2<R>) * ((long long)tile * TX);
-    const size_t cstride = (size_t)sizeof(C2<R>) * a.comp_src;
-    const size_t rstride = (size_t)sizeof(C2<R>) * T * a.s_col;
-    const unsigned voff = (unsigned)(sizeof(C2<R>) * ((size_t)j * a.s_col + c));
-    // lanes past nx load the last valid column and store nothing
-    const unsigned loff = (unsigned)(sizeof(C2<R>) * ((size_t)j * a.s_col + min(c, a.nx - 1 - tile * TX)));
-    // the block's TX columns lie in one tile of the G layout (gtx a multiple of TX)
-    const int xg = a.x0 + tile * TX;
-    const int cg = xg % a.gtx + c;
-    const char* g = reinterpret_cast<const char*>(a.green) +
-                    sizeof(R) * ((long long)y0 * a.gntx + xg / a.gtx) * (M / 2 + 1) * a.gtx;
-    const R* sym = reinterpret_cast<const R*>(rk.sym);
-    const R kx = sym[rk.off[0] + a.x0 + min(x, a.nx - 1)];
-    // the twiddle table copied to LDS: seven LDS reads per radix-8 stage instead of three loads and
-    // four complex products (the FP32 pass runs seven column FFTs per column set)
-    for (int i = threadIdx.x; i < M; i += TX * M / 8) ltw[i] = reinterpret_cast<const C2<R>*>(a.tw)[i];
-    __syncthreads();
-    const C2<R>* tw = ltw;
-    for (int s = 0; s < 2; ++s) {
-        const int y = s == 0 ? y0 : y1;
-        char* b = base + (size_t)sizeof(C2<R>) * ((long long)y * a.s_other_src);
-        const R ky = sym[rk.off[1] + y];
-        // Two sets of NV values live at a time (u = i K x psi, psi = G w). The pass is in place and
-        // every w_c enters two components of u, so the components are written to the slot of an
-        // input this block already holds as psi: u_z to slot x, u_y to slot z, u_x to slot y (w_y is
-        // read and transformed twice); the inverse y pass reads component c from slot (c + 1) mod 3.
-        C2<R> p[NV], q[NV];
-        auto load = [&](C2<R>* u, int cc) {
-#pragma unroll
-            for (int i = 0; i < NV; ++i) {
-                const int row = j + i * T;
-                u[i] = row < a.nin ? *reinterpret_cast<const C2<R>*>(b + cc * cstride + i * rstride + loff) : C2<R>{0, 0};
-            }
-        };
-        auto store = [&](int cc, const C2<R>* u) {
-            if (!live) return;
-#pragma unroll
-            for (int i = 0; i < NV; ++i) {
-                const int row = j + i * T;
-                if (row < a.nout) *reinterpret_cast<C2<R>*>(b + cc * cstride + i * rstride + voff) = u[i];
-            }
-        };
-        auto psi = [&](C2<R>* u) {   // forward transform, times normfact G (re-read for each use: fewer live registers)
-            column_fft<R, M, true, TX, false, true>(u, lds + c, j, tw);
-#pragma unroll
-            for (int i = 0; i < NV; ++i) {
-                const int kz = j + i * T;
-                const R gk = *reinterpret_cast<const R*>(g + (unsigned)(sizeof(R) * (min(kz, M - kz) * a.gtx + cg)));
-                u[i] = {u[i].x * gk, u[i].y * gk};
-            }
-        };
-        auto kz_of = [&](int i) { return sym[rk.off[2] + j + i * T]; };
-        load(p, 0);
-        load(q, 1);
-        psi(p);   // psi_x
-        psi(q);   // psi_y
-#pragma unroll
-        for (int i = 0; i < NV; ++i) {   // u_z = i (kx psi_y - ky psi_x)
-            const C2<R> cz = {kx * q[i].x - ky * p[i].x, kx * q[i].y - ky * p[i].y};
-            q[i] = {-cz.y, cz.x};
-        }
-        column_fft<R, M, false, TX, false, true>(q, lds + c, j, tw);
-        store(0, q);
-        load(q, 2);
-        psi(q);   // psi_z
-#pragma unroll
-        for (int i = 0; i < NV; ++i) {   // u_y = i (kz psi_x - kx psi_z)
-            const R kz = kz_of(i);
-            const C2<R> cy = {kz * p[i].x - kx * q[i].x, kz * p[i].y - kx * q[i].y};
-            p[i] = {-cy.y, cy.x};
-        }
-        column_fft<R, M, false, TX, false, true>(p, lds + c, j, tw);
-        store(2, p);
-        load(p, 1);
-        psi(p);   // psi_y again
-#pragma unroll
-        for (int i = 0; i < NV; ++i) {   // u_x = i (ky psi_z - kz psi_y)
-            const R kz = kz_of(i);
-            const C2<R> cx = {ky * q[i].x - kz * p[i].x, ky * q[i].y - kz * p[i].y};
-            p[i] = {-cx.y, cx.x};
-        }
-        column_fft<R, M, false, TX, false, true>(p, lds + c, j, tw);
-        store(1, p);
-        if (!pair) break;   // uniform over the block
-    }
-}
-
-template <typename R, int M, int TX>
-__device__ __forceinline__ void z_rot_body(const ColArgs& a, const RotK& rk, C2<R>* lds, C2<R>* ltw, Blk bk) {
-    if constexpr (sizeof(R) == 4) z_rot_body2<R, M, TX>(a, rk, lds, ltw, bk);
-    else z_rot_body3<R, M, TX>(a, rk, lds, bk);
-}
-
-// at most 256 registers per lane (two waves per SIMD): the three components need 250-285
-// (FP64), and the few that spill cost less than halving the waves (513^3 x 3 solve: 34.0 ->
-// 29.8 ms)
-struct ZRotArgs {
-    ColArgs a;
-    RotK rk;
-};
-template <typename R, int M, int TX>
-struct z_rot {
-    using Args = ZRotArgs;
-    static constexpr int NT = TX * M / 8;
-    static constexpr int kWaves = 2;
-    static __device__ __forceinline__ void run(const ZRotArgs& z, Blk bk) {
-        __shared__ C2<R> lds[M * TX];
-        __shared__ C2<R> ltw[sizeof(R) == 4 ? M : 1];   // FP32: the twiddle table
-        z_rot_body<R, M, TX>(z.a, z.rk, lds, ltw, bk);
-    }
-};
 
 // ---------------------------------------------------------------------------
 // x rows: r2c of the zero-padded real row (length M = 2*H) through the packed
@@ -1037,21 +786,6 @@ void col_dispatch(int M, const ColArgs& a, int comps, int zsched, hipStream_t st
     }
 }
 
-template <typename R, int TX>
-void launch_rot(int M, const ColArgs& a, const RotK& rk, hipStream_t st) {
-    dim3 grid(((a.nx + TX - 1) / TX) * (a.gmy / 2 + 1), 1);
-    switch (M) {
-        case 32: launch_k<z_rot<R, 32, TX>>(grid, dim3(TX * 4), 0, st, {a, rk}); break;
-        case 64: launch_k<z_rot<R, 64, TX>>(grid, dim3(TX * 8), 0, st, {a, rk}); break;
-        case 128: launch_k<z_rot<R, 128, TX>>(grid, dim3(TX * 16), 0, st, {a, rk}); break;
-        case 256: launch_k<z_rot<R, 256, TX>>(grid, dim3(TX * 32), 0, st, {a, rk}); break;
-        case 512: launch_k<z_rot<R, 512, TX>>(grid, dim3(TX * 64), 0, st, {a, rk}); break;
-        case 1024: launch_k<z_rot<R, 1024, TX>>(grid, dim3(TX * 128), 0, st, {a, rk}); break;
-        default: fail("unsupported column length %d", M);
-    }
-    HIP_CHECK(hipGetLastError());
-}
-
 template <typename R, int MODE>
 void row_launch(bool fwd, int H, const RowArgs& a, int comps, hipStream_t st) {
 #define FLUPS_ROW(HH, RR)                                                                                   \
@@ -1173,19 +907,10 @@ void run_fast(FastPlan* f, void* s0, void* s1, const double* rhs, double* field,
         z.x0 = x0;
         z.gntx = (f->nx + f->gtx - 1) / f->gtx;
         if (type == 1) {
-            // rotational pass: all three components per block, tile width of the Green's layout
+            // rotational pass: all three components per block
             FLUPS_REQUIRE(f->lda == 3, "the rotational solve needs lda = 3");
             z.gtx = f->gtx;
-            if (M2 == 1024 && f->gtx == TX / 2 && sizeof(R) == 8) {
-                // M2 = 1024, FP64: the Green's layout width, four columns of 64-byte rows per block
-                // of 512 threads (two columns of 32-byte rows: 28.5 instead of 27.8 ms at 513^3 x 3);
-                // FP32 keeps a quarter of the stage tile (eight columns would need 1024 threads of
-                // 157 registers)
-                launch_rot<R, TX / 2>(M2, z, f->rot, st);
-            } else if (M2 == 1024 && f->gtx == TX / 2) launch_rot<R, TX / 4>(M2, z, f->rot, st);
-            else if (f->gtx == TX) launch_rot<R, TX>(M2, z, f->rot, st);
-            else if (f->gtx == TX / 2) launch_rot<R, TX / 2>(M2, z, f->rot, st);
-            else launch_rot<R, (TX >= 8 ? TX / 4 : 1)>(M2, z, f->rot, st);
+            launch_z_rot<R>(M2, z, f->rot, st);
         } else {
             col_dispatch<R, TX, true, true>(M2, z, f->lda, f->zsched, st);
         }
@@ -1193,7 +918,6 @@ void run_fast(FastPlan* f, void* s0, void* s1, const double* rhs, double* field,
         // 4. y inverse: S1 -> columns [x0, x0 + w) of S0, keep N1
         ColArgs b = a;
         b.rev = (f->order >> 1) & 1;
-        b.crot = (type == 1 && sizeof(R) == 4) ? 1 : 0;   // FP32 z_rot leaves u_c in slot (c + 1) mod 3
         b.src = s1;
         b.dst = reinterpret_cast<char*>(s0) + es * x0;
         b.s_col = f->ldxs;

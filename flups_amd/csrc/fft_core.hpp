@@ -87,14 +87,15 @@ __device__ __forceinline__ void dft4(C2<R>& a0, C2<R>& a1, C2<R>& a2, C2<R>& a3)
     a1 = cadd(d0, d1);
     a3 = csub(d0, d1);
 }
-// HIN: v[4..7] are zero (zero-padded input) and are not read
-template <typename R, bool FWD, bool HIN = false>
+// HIN = 1: v[4..7] are zero (zero-padded input) and are not read; 2: v[5..7] (one value more: node-centred)
+template <typename R, bool FWD, int HIN = 0>
 __device__ __forceinline__ void dft8(C2<R>* v) {
     const R h = (R)0.70710678118654752440;
     // radix-2 split into even/odd halves, then 4-point DFTs
     C2<R> e0, e1, e2, e3, o0, o1, o2, o3;
     if (HIN) {
-        e0 = o0 = v[0];
+        e0 = HIN == 2 ? cadd(v[0], v[4]) : v[0];
+        o0 = HIN == 2 ? csub(v[0], v[4]) : v[0];
         e1 = o1 = v[1];
         e2 = o2 = v[2];
         e3 = o3 = v[3];
@@ -148,12 +149,17 @@ __device__ __forceinline__ int lslot(int e) { return ES > 0 ? e * ES : e + (e >>
 // Full column FFT of length M held by a team of T = M/8 threads (j = 0..T-1).
 // On entry v[i] = x[j + i*T]; on exit v[i] = X[j + i*T]. lds points at the
 // column (element e at lds[lslot<ES>(e)]); the whole block must call this together.
-// HIN: the upper half of the input is zero (v[4..7] not read). Outputs the caller
+// HIN = 1: the upper half of the input is zero (v[4..7] not read), 2: but for v[4]. Outputs the caller
 // never uses (the upper half of a truncated inverse) are removed by the compiler.
 // LTW: tw is a copy of the table in LDS, and each radix-8 stage reads its seven
 // twiddles w^q from it (seven LDS reads instead of three table loads and four
 // complex products: fewer VALU instructions for kernels bound by them).
-template <typename R, int M, bool FWD, int ES, bool HIN = false, bool LTW = false>
+// PP = 0 or 1: two LDS buffers, lds and lds + M ES, taken in turn by the exchanges, the first one of
+// this call in buffer PP: one barrier per exchange instead of two, for a kernel whose registers
+// leave the LDS half empty. The next call starts at (PP + column_exchanges(M)) & 1, with no barrier
+// between the calls. PP = -1: one buffer.
+constexpr int column_exchanges(int m) { return m <= 8 ? 0 : 1 + column_exchanges((m + 7) / 8); }
+template <typename R, int M, bool FWD, int ES, int HIN = 0, bool LTW = false, int PP = -1>
 __device__ __forceinline__ void column_fft(C2<R>* v, C2<R>* lds, int j, const C2<R>* tw) {
     constexpr int T = M / 8;
     // table entries w, w^2, w^4 of the next radix-8 stage, loaded one stage ahead
@@ -162,8 +168,10 @@ __device__ __forceinline__ void column_fft(C2<R>* v, C2<R>* lds, int j, const C2
     // competes with the data loads: FP32 z pass 184 -> 236 us at 256^3)
     C2<R> r1 = {1, 0}, r2 = {1, 0}, r4 = {1, 0};
     int span = 1;
+    C2<R>* const bank = lds;
 #pragma unroll
     for (int st = 0; st < 8; ++st) {
+        if (PP >= 0) lds = bank + (((PP + st + 1) & 1) ? M * ES : 0);   // read: the buffer of the previous exchange
         // stages of radix 8 while 8*span <= M, then one radix 4 or 2 stage
         if (span >= M) break;
         const int P = (span * 8 <= M) ? 8 : (M / span);
@@ -199,10 +207,11 @@ __device__ __forceinline__ void column_fft(C2<R>* v, C2<R>* lds, int j, const C2
 #pragma unroll
                 for (int q = 1; q < 8; ++q) v[q] = cmul(v[q], tw8[q]);
             }
-            if (HIN && span == 1) dft8<R, FWD, true>(v);
+            if (HIN && span == 1) dft8<R, FWD, HIN>(v);
             else dft8<R, FWD>(v);
             if (span * 8 < M) {
-                __syncthreads();   // everyone has read this stage's inputs
+                if (PP >= 0) lds = bank + (((PP + st) & 1) ? M * ES : 0);
+                else __syncthreads();   // everyone has read this stage's inputs
                 const int base = (j / span) * span * 8 + k;
 #pragma unroll
                 for (int u = 0; u < 8; ++u) lds[lslot<ES>(base + u * span)] = v[u];
