@@ -138,6 +138,21 @@ struct SmoothZArgs {
     SmoothPlan sm;
 };
 
+// the same with the curl of three components (smooth_rot.hip)
+struct SmoothRotArgs {
+    void* d = nullptr;           // the three components before the transform, in place: complex, x fastest
+    const void* g = nullptr;     // normfact G, [y'][tile][kz'][gtx]
+    const double* tw = nullptr;  // M-point twiddle table
+    const double* sym = nullptr; // derivative symbols by mode index: x, y, z at off[0], off[1], off[2]
+    int off[3] = {0, 0, 0};
+    int nx = 1, nother = 1, nin = 1, tx = 4;
+    int gtx = 4, gntx = 1;       // tiles of G
+    int mirror = 0;              // 1: the rows y and nother - y share their G
+    int f32 = 0;                 // data and G stored as float (FP64 arithmetic)
+    long long s_col = 1, s_other = 1, comp = 0;
+    SmoothPlan sm;
+};
+
 // the last direction of the general path as one r2c -> normfact G -> c2r launch (rowpass.hip):
 // col_rz, real columns along the last dimension, pairs of neighbours along x; row_rz, real rows
 // along x (x the last direction); nin real values per column / row, transform length M

@@ -995,6 +995,8 @@ bool row_rz_len_ok(int M);
 bool split_pq(int n, int& pf, int& q);
 int smooth_z_tile(int M, bool f32);                          // smooth.hip
 void launch_smooth_z(const SmoothZArgs& A, hipStream_t s);
+int smooth_rot_tile(int M, bool f32);                        // smooth_rot.hip
+void launch_smooth_rot(const SmoothRotArgs& A, hipStream_t s);
 
 struct HybridZ {
     int M = 0, nx = 0, ny = 0, nz = 0, lda = 1, gtx = 8;
@@ -1010,6 +1012,8 @@ struct HybridZ {
     void* green = nullptr;   // normfact * Re G, [y'][tile][kz'][gtx]
     void* tw = nullptr;      // (M / pf)-point table
     void* twm = nullptr;     // M-point table (pf 3)
+    int rtx = 0;             // columns per block of the fused rotational pass (0: none)
+    double* sym = nullptr;   // its derivative symbols: x, y, z
     size_t dev_bytes = 0;
     double bytes = 0;        // algorithmic bytes of one launch
 };
@@ -1145,8 +1149,30 @@ HybridZ* make_hybrid_z(SolverImpl& s) {
             HIP_CHECK(hipMemcpy(h->twm, tm.data(), tm.size() * sizeof(double), hipMemcpyHostToDevice));
             h->dev_bytes += tm.size() * sizeof(double);
         }
+        // the rotational pass: every direction unbounded or periodic, so that each derivative is i K with
+        // the same real K for the three components
+        bool rot = nd == 3 && s.lda_ == 3 && s.odiff_ != NOD;
+        RotK rk{};
+        for (int i = 0; i < nd && rot; ++i) {
+            const DirPlan& p = s.fwd_[i];
+            rot = (p.type == UNBUNB || p.type == PERPER) && p.koffset == 0.0;
+            for (int c = 0; c < 3; ++c) rot = rot && s.bwdd_[i].imult[c] == p.imult[c];
+            rk.kfact[p.dim] = p.kfact;
+            rk.symstart[p.dim] = p.symstart;
+            rk.h[p.dim] = s.h_[p.dim];
+        }
+        if (rot && (h->rtx = smooth_rot_tile(M, f32)) > 0) {
+            rk.order = s.odiff_;
+            std::vector<double> t3;
+            for (int d = 0; d < 3; ++d)
+                for (int i = 0; i < sp.n[d]; ++i) t3.push_back(rot_symbol(rk, d, i));
+            HIP_CHECK(hipMalloc(&h->sym, t3.size() * sizeof(double)));
+            HIP_CHECK(hipMemcpy(h->sym, t3.data(), t3.size() * sizeof(double), hipMemcpyHostToDevice));
+            h->dev_bytes += t3.size() * sizeof(double);
+        }
         HIP_CHECK(hipStreamSynchronize(s.stream_));
     } catch (...) {
+        (void)hipFree(h->sym);
         (void)hipFree(h->green);
         (void)hipFree(h->tw);
         (void)hipFree(h->twm);
@@ -1164,8 +1190,10 @@ void destroy_hybrid_z(HybridZ* h) {
     (void)hipFree(h->tw);
     (void)hipFree(h->twm);
     (void)hipFree(h->twn);
+    (void)hipFree(h->sym);
     delete h;
 }
+bool hybrid_runs(const HybridZ* h, int type) { return type == 0 || h->rtx > 0; }
 size_t hybrid_device_bytes(const HybridZ* h) { return h->dev_bytes; }
 double hybrid_bytes(const HybridZ* h) { return h->bytes; }
 
@@ -1335,7 +1363,31 @@ void hybrid_z_t(const HybridZ* h, void* data, hipStream_t st) {
     // half-width tiles (schedule bit 2), XCD-grouped; M = 1024 is already half width
     col_dispatch<double, 8, true, true, S>(h->M, z, h->lda, 4 | 16, st);
 }
-void hybrid_z(const HybridZ* h, void* data, hipStream_t st) {
+// type 1: the rotational pass (hybrid_runs)
+void hybrid_z(const HybridZ* h, void* data, int type, hipStream_t st) {
+    if (type != 0) {
+        SmoothRotArgs A;
+        A.d = data;
+        A.g = h->green;
+        A.tw = static_cast<const double*>(h->pf > 1 ? h->twm : h->tw);
+        A.sym = h->sym;
+        A.off[1] = h->nx;
+        A.off[2] = h->nx + h->ny;
+        A.nx = h->nx;
+        A.nother = h->ny;
+        A.nin = h->nz;
+        A.tx = h->rtx;
+        A.gtx = h->gtx;
+        A.gntx = (h->nx + h->gtx - 1) / h->gtx;
+        A.mirror = h->pair;
+        A.f32 = h->f32;
+        A.s_col = (long long)h->nx * h->ny;
+        A.s_other = h->nx;
+        A.comp = (long long)h->nx * h->ny * h->nz;
+        smooth_plan(h->M, A.sm);
+        launch_smooth_rot(A, st);
+        return;
+    }
     if (h->f32) hybrid_z_t<float>(h, data, st);
     else hybrid_z_t<double>(h, data, st);
 }

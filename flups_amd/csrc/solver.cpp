@@ -63,7 +63,8 @@ HybridZ* make_hybrid_z(SolverImpl& s);
 void destroy_hybrid_z(HybridZ* h);
 size_t hybrid_device_bytes(const HybridZ* h);
 double hybrid_bytes(const HybridZ* h);
-void hybrid_z(const HybridZ* h, void* data, hipStream_t st);
+bool hybrid_runs(const HybridZ* h, int type);
+void hybrid_z(const HybridZ* h, void* data, int type, hipStream_t st);
 void fast_schedule(const FastPlan* f, int out[3]);
 double fast_bytes(const FastPlan* f);
 void fast_autotune(FastPlan* f, double* out, const double* in, const View& uin, const View& uout, const double* dgreen,
@@ -841,7 +842,7 @@ void SolverImpl::backward_passes(const void* spec, const View& uout, bool diff) 
 }
 
 void SolverImpl::solve_generic(double* field, const double* rhs, int type) {
-    if (hybrid_ && type == 0) {
+    if (hybrid_ && hybrid_runs(hybrid_, type)) {
         // general passes for the first directions, the last one fused with the multiply
         const View uin = user_view(const_cast<double*>(rhs)), uout = user_view(field);
         for (int ip = 0; ip < ndim_ - 1; ++ip) {
@@ -852,10 +853,10 @@ void SolverImpl::solve_generic(double* field, const double* rhs, int type) {
             for (int c = 0; c < lda_; ++c) run_pass(pass_desc(p, c, true, src, dst, hat_[ip], stage_[ip], p.fieldstart, 0));
         }
         pmark("fftw forward");
-        hybrid_z(hybrid_, dstage_[ndim_ - 2], stream_);
+        hybrid_z(hybrid_, dstage_[ndim_ - 2], type, stream_);
         pmark("fftw + domagic (last direction fused)");
         for (int ip = ndim_ - 2; ip >= 0; --ip) {
-            const DirPlan& p = bwd_[ip];
+            const DirPlan& p = type != 0 ? bwdd_[ip] : bwd_[ip];
             const View src = dense_view(dstage_[ip], stage_[ip], ses_);
             const View dst = (ip == 0) ? uout : dense_view(dstage_[ip - 1], stage_[ip - 1], ses_);
             SameStage same;
@@ -1252,12 +1253,13 @@ double SolverImpl::algorithmic_bytes(int type) const {
     const double w = sizeof(double);
     const double user = (double)phys_.nglob[0] * phys_.nglob[1] * phys_.nglob[2] * lda_;
     double b = 0;
-    const int nfull = (hybrid_ && type == 0) ? ndim_ - 1 : ndim_;
+    const bool fused = hybrid_ && hybrid_runs(hybrid_, type);
+    const int nfull = fused ? ndim_ - 1 : ndim_;
     for (int ip = 0; ip < nfull; ++ip) {
         const double in = ip == 0 ? user : (double)stage_[ip - 1].count();
         b += 2.0 * w * (in + (double)stage_[ip].count());   // forward pass and its backward mirror
     }
-    if (hybrid_ && type == 0) return b + hybrid_bytes(hybrid_);
+    if (fused) return b + hybrid_bytes(hybrid_);
     const Shape& sp = stage_[ndim_ - 1];
     b += w * (2.0 * (double)sp.count() + (double)gpost_[ndim_ - 1].count());
     (void)type;
