@@ -95,7 +95,7 @@ struct SmoothPlan {
 };
 bool smooth_plan(int M, SmoothPlan& p);   // smooth.hip; false when M has another prime factor or is out of range
 
-// everything one launch of the generic pencil kernel needs (one component)
+// everything one launch of a pencil kernel needs: one component, or all lda of them (the grid's y)
 struct PassDesc {
     int d = 0;
     int op = OP_NONE, sign = FWD;
@@ -123,6 +123,12 @@ struct PassDesc {
     int nt = 0;             // row r2r kernel: its vector accesses are non-temporal (both arrays 128 MiB or more)
     const double* aux = nullptr;   // fast kernels: pre / post twiddle table
     SmoothPlan sm;          // M > 0: kernels of smooth.hip, their stages (sm.T threads per pencil, ppb pencils per block)
+    int lda = 1;                        // components of the launch, src_c / dst_c reals apart
+    long long src_c = 0, dst_c = 0;
+    template <typename T>
+    __host__ __device__ const T* from(int c) const { return reinterpret_cast<const T*>(src) + c * src_c; }
+    template <typename T>
+    __host__ __device__ T* to(int c) const { return reinterpret_cast<T*>(dst) + c * dst_c; }
 };
 
 // the last direction of the general path, c2c of a smooth length, with the multiply (smooth.hip)

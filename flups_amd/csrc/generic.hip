@@ -162,7 +162,7 @@ struct generic_pass {
                 const int ks = k - P.gshift;
                 const long long idx = (long long)min(max(ks, 0), last) * P.src_s[d] + (long long)ja * P.src_s[P.fa] +
                                       (long long)jb * P.src_s[P.fb];
-                const TI* sp = reinterpret_cast<const TI*>(P.src) + idx * P.src_nf;
+                const TI* sp = P.from<TI>(blk.y) + idx * P.src_nf;
                 const double x0 = (double)sp[0], x1 = nfi > 1 ? (double)sp[1] : 0.0;
                 const bool in = ks >= 0 && ks < P.src_nd;
                 return cd{in ? x0 : 0.0, in ? x1 : 0.0};
@@ -331,7 +331,7 @@ struct generic_pass {
                 const int ja = g % P.na, jb = g / P.na;
                 const double* v = pb + (size_t)pen * len + (size_t)kt * P.nf_out;
                 const long long idx = (long long)k * P.dst_s[d] + (long long)ja * P.dst_s[P.fa] + (long long)jb * P.dst_s[P.fb];
-                TO* dp = reinterpret_cast<TO*>(P.dst) + idx * nfo;
+                TO* dp = P.to<TO>(blk.y) + idx * nfo;
                 for (int c = 0; c < nfo; ++c) dp[c] = (TO)v[c];
             }
         }
@@ -354,10 +354,10 @@ void launch_generic(const PassDesc& P, hipStream_t s) {
     // threads: enough for one element (or butterfly) each of the block's pencils, whole waves, at most 256
     const int work = P.ppb * std::max(P.M, P.pen_in);
     const int threads = std::min(256, std::max(64, (work + 63) / 64 * 64));
-    if (!P.src_f32 && !P.dst_f32) launch_k<generic_pass<double, double>>(dim3(blocks), dim3(threads), lds, s, P);
-    else if (!P.src_f32) launch_k<generic_pass<double, float>>(dim3(blocks), dim3(threads), lds, s, P);
-    else if (P.dst_f32) launch_k<generic_pass<float, float>>(dim3(blocks), dim3(threads), lds, s, P);
-    else launch_k<generic_pass<float, double>>(dim3(blocks), dim3(threads), lds, s, P);
+    if (!P.src_f32 && !P.dst_f32) launch_k<generic_pass<double, double>>(dim3(blocks, P.lda), dim3(threads), lds, s, P);
+    else if (!P.src_f32) launch_k<generic_pass<double, float>>(dim3(blocks, P.lda), dim3(threads), lds, s, P);
+    else if (P.dst_f32) launch_k<generic_pass<float, float>>(dim3(blocks, P.lda), dim3(threads), lds, s, P);
+    else launch_k<generic_pass<float, double>>(dim3(blocks, P.lda), dim3(threads), lds, s, P);
     HIP_CHECK(hipGetLastError());
 }
 

@@ -122,8 +122,8 @@ struct pen_r2r {
             jb = gg / P.na;
         }
         const int k1 = tt / T, j = tt % T;   // team and thread in the team
-        const TI* src = reinterpret_cast<const TI*>(P.src) + (long long)ja * P.src_s[P.fa] + (long long)jb * P.src_s[P.fb];
-        TO* dst = reinterpret_cast<TO*>(P.dst) + (long long)ja * P.dst_s[P.fa] + (long long)jb * P.dst_s[P.fb];
+        const TI* src = P.from<TI>(blk.y) + (long long)ja * P.src_s[P.fa] + (long long)jb * P.src_s[P.fb];
+        TO* dst = P.to<TO>(blk.y) + (long long)ja * P.dst_s[P.fa] + (long long)jb * P.dst_s[P.fb];
         const long long sd = P.src_s[P.d], dd = P.dst_s[P.d];
         C2<double>* row = COL ? lds + rl : lds + rl * HP;                                    // complex view
         double* rdb = COL ? reinterpret_cast<double*>(lds) + rl : reinterpret_cast<double*>(row);   // real view
@@ -325,8 +325,8 @@ struct row_rc {
         const bool live = g < P.n1 * P.n2;
         const int gg = live ? g : 0;   // dead rows read pencil 0 and store nothing
         const int ja = gg % P.na, jb = gg / P.na;
-        const TI* src = reinterpret_cast<const TI*>(P.src) + (long long)ja * P.src_s[P.fa] * P.src_nf + (long long)jb * P.src_s[P.fb] * P.src_nf;
-        TO* dst = reinterpret_cast<TO*>(P.dst) + (long long)ja * P.dst_s[P.fa] * P.dst_nf + (long long)jb * P.dst_s[P.fb] * P.dst_nf;
+        const TI* src = P.from<TI>(blk.y) + (long long)ja * P.src_s[P.fa] * P.src_nf + (long long)jb * P.src_s[P.fb] * P.src_nf;
+        TO* dst = P.to<TO>(blk.y) + (long long)ja * P.dst_s[P.fa] * P.dst_nf + (long long)jb * P.dst_s[P.fb] * P.dst_nf;
         C2<double>* row = lds + rl * HP;
         double* rd = reinterpret_cast<double*>(row);
         const C2<double>* tw = reinterpret_cast<const C2<double>*>(P.tw);    // Q-point table
@@ -435,10 +435,10 @@ struct col_real {
         const int d = P.d;
         const long long sr = FWD ? P.src_s[d] : P.dst_s[d];       // row stride of the real array
         const long long sc = FWD ? P.dst_s[d] : P.src_s[d];       // row stride of the complex array
-        const TI* rsrc = reinterpret_cast<const TI*>(P.src) + (long long)jb * P.src_s[P.fb] + xa;          // FWD: real source
-        TO* rdst = reinterpret_cast<TO*>(P.dst) + (long long)jb * P.dst_s[P.fb] + xa;                    // !FWD: real destination
-        const TI* csrc = reinterpret_cast<const TI*>(P.src) + 2 * ((long long)jb * P.src_s[P.fb] + xa);   // !FWD: complex source
-        TO* cdst = reinterpret_cast<TO*>(P.dst) + 2 * ((long long)jb * P.dst_s[P.fb] + xa);             // FWD: complex destination
+        const TI* rsrc = P.from<TI>(blk.y) + (long long)jb * P.src_s[P.fb] + xa;          // FWD: real source
+        TO* rdst = P.to<TO>(blk.y) + (long long)jb * P.dst_s[P.fb] + xa;                    // !FWD: real destination
+        const TI* csrc = P.from<TI>(blk.y) + 2 * ((long long)jb * P.src_s[P.fb] + xa);   // !FWD: complex source
+        TO* cdst = P.to<TO>(blk.y) + 2 * ((long long)jb * P.dst_s[P.fb] + xa);             // FWD: complex destination
         const bool hasb = lb;   // a real partner column exists
         const C2<double>* tw = reinterpret_cast<const C2<double>*>(P.tw);    // Q-point table
         const C2<double>* twm = reinterpret_cast<const C2<double>*>(P.aux);  // M-point table (PF > 1)
@@ -697,8 +697,8 @@ struct col_c2c {
         int ja = tile * TX + c;
         const bool live = ja < P.na;
         if (!live) ja = P.na - 1;   // dead columns read the last one and store nothing
-        const C2<TI>* src = reinterpret_cast<const C2<TI>*>(P.src) + (long long)ja * P.src_s[P.fa] + (long long)jb * P.src_s[P.fb];
-        C2<TO>* dst = reinterpret_cast<C2<TO>*>(P.dst) + (long long)ja * P.dst_s[P.fa] + (long long)jb * P.dst_s[P.fb];
+        const C2<TI>* src = reinterpret_cast<const C2<TI>*>(P.from<TI>(blk.y)) + (long long)ja * P.src_s[P.fa] + (long long)jb * P.src_s[P.fb];
+        C2<TO>* dst = reinterpret_cast<C2<TO>*>(P.to<TO>(blk.y)) + (long long)ja * P.dst_s[P.fa] + (long long)jb * P.dst_s[P.fb];
         const long long sd = P.src_s[P.d], dd = P.dst_s[P.d];
         C2<double> v[NV];
     #pragma unroll
@@ -743,8 +743,8 @@ struct row_c2c {
         const bool live = g < P.n1 * P.n2;
         const int gg = live ? g : 0;   // dead rows read pencil 0 and store nothing
         const int ja = gg % P.na, jb = gg / P.na;
-        const C2<TI>* src = reinterpret_cast<const C2<TI>*>(P.src) + (long long)ja * P.src_s[P.fa] + (long long)jb * P.src_s[P.fb];
-        C2<TO>* dst = reinterpret_cast<C2<TO>*>(P.dst) + (long long)ja * P.dst_s[P.fa] + (long long)jb * P.dst_s[P.fb];
+        const C2<TI>* src = reinterpret_cast<const C2<TI>*>(P.from<TI>(blk.y)) + (long long)ja * P.src_s[P.fa] + (long long)jb * P.src_s[P.fb];
+        C2<TO>* dst = reinterpret_cast<C2<TO>*>(P.to<TO>(blk.y)) + (long long)ja * P.dst_s[P.fa] + (long long)jb * P.dst_s[P.fb];
         C2<double>* row = lds + rl * HP;
         const int last = max(P.src_nd - 1, 0);
         staged_gather<8>(tt, TT, M, [&](int k) {
@@ -787,8 +787,8 @@ struct col_c2c_team {
         int ja = tile * TX + c;
         const bool live = ja < P.na;
         if (!live) ja = P.na - 1;   // dead columns read the last one and store nothing
-        const C2<TI>* src = reinterpret_cast<const C2<TI>*>(P.src) + (long long)ja * P.src_s[P.fa] + (long long)jb * P.src_s[P.fb];
-        C2<TO>* dst = reinterpret_cast<C2<TO>*>(P.dst) + (long long)ja * P.dst_s[P.fa] + (long long)jb * P.dst_s[P.fb];
+        const C2<TI>* src = reinterpret_cast<const C2<TI>*>(P.from<TI>(blk.y)) + (long long)ja * P.src_s[P.fa] + (long long)jb * P.src_s[P.fb];
+        C2<TO>* dst = reinterpret_cast<C2<TO>*>(P.to<TO>(blk.y)) + (long long)ja * P.dst_s[P.fa] + (long long)jb * P.dst_s[P.fb];
         const long long sd = P.src_s[P.d], dd = P.dst_s[P.d];
         // all eight loads (clamped addresses, zero selected afterwards) before the LDS writes
         const int last = max(P.src_nd - 1, 0);
@@ -823,7 +823,7 @@ template <int PF, int Q, int R, bool COL, typename TI, typename TO>
 void launch_pen_h(const PassDesc& P, hipStream_t s) {
     const int npen = P.n1 * P.n2;
     const int nb = COL ? ((P.na + R - 1) / R) * (npen / P.na) : (npen + R - 1) / R;
-    dim3 grid(nb);
+    dim3 grid(nb, P.lda);
     dim3 block(R * PF * Q / 8);
     switch (P.kind) {
         case REDFT10: launch_k<pen_r2r<PF, Q, R, REDFT10, COL, TI, TO>>(grid, block, 0, s, P); break;
@@ -854,7 +854,7 @@ void launch_pen_pf(int q, const PassDesc& P, hipStream_t s) {
 
 template <int PF, int Q, int ROWS, typename TI, typename TO>
 void launch_row_rc_h(const PassDesc& P, hipStream_t s) {
-    dim3 grid((P.n1 * P.n2 + ROWS - 1) / ROWS);
+    dim3 grid((P.n1 * P.n2 + ROWS - 1) / ROWS, P.lda);
     dim3 block(ROWS * PF * Q / 8);
     if (P.op == OP_R2C) launch_k<row_rc<PF, Q, ROWS, true, TI, TO>>(grid, block, 0, s, P);
     else launch_k<row_rc<PF, Q, ROWS, false, TI, TO>>(grid, block, 0, s, P);
@@ -877,7 +877,7 @@ void launch_col_real_m(const PassDesc& P, hipStream_t s) {
     const int npair = (P.na + 1) / 2;
     const int ntile = (npair + TX - 1) / TX;
     const int nb = P.n1 * P.n2 / P.na;
-    dim3 grid(ntile * nb);
+    dim3 grid(ntile * nb, P.lda);
     if (P.op == OP_R2C) launch_k<col_real<PF, Q, TX, true, TI, TO>>(grid, dim3(TX * Q / 8), 0, s, P);
     else launch_k<col_real<PF, Q, TX, false, TI, TO>>(grid, dim3(TX * Q / 8), 0, s, P);
 }
@@ -899,7 +899,7 @@ template <int PF, int Q, int TX, typename TI, typename TO>
 void launch_col_c2c_m(const PassDesc& P, hipStream_t s) {
     constexpr int M = PF * Q;
     const int ntile = (P.na + TX - 1) / TX;
-    dim3 grid(ntile * (P.n1 * P.n2 / P.na));
+    dim3 grid(ntile * (P.n1 * P.n2 / P.na), P.lda);
     dim3 block(TX * Q / 8);
     const bool hin = P.gshift == 0 && P.src_nd <= M / 2, hout = P.sshift == 0 && P.dst_nd <= M / 2;
     if (P.sign == FWD) {
@@ -913,7 +913,7 @@ void launch_col_c2c_m(const PassDesc& P, hipStream_t s) {
 template <int PF, int Q, int TX, typename TI, typename TO>
 void launch_col_c2c_t(const PassDesc& P, hipStream_t s) {
     const int ntile = (P.na + TX - 1) / TX;
-    dim3 grid(ntile * (P.n1 * P.n2 / P.na));
+    dim3 grid(ntile * (P.n1 * P.n2 / P.na), P.lda);
     dim3 block(TX * PF * Q / 8);
     if (P.sign == FWD) launch_k<col_c2c_team<PF, Q, TX, true, TI, TO>>(grid, block, 0, s, P);
     else launch_k<col_c2c_team<PF, Q, TX, false, TI, TO>>(grid, block, 0, s, P);
@@ -921,7 +921,7 @@ void launch_col_c2c_t(const PassDesc& P, hipStream_t s) {
 template <int PF, int Q, typename TI, typename TO>
 void launch_row_c2c_h(const PassDesc& P, hipStream_t s) {
     constexpr int ROWS = 2048 / (PF * Q) > 0 ? 2048 / (PF * Q) : 1;   // about 256 threads, 36 KB of LDS
-    dim3 grid((P.n1 * P.n2 + ROWS - 1) / ROWS);
+    dim3 grid((P.n1 * P.n2 + ROWS - 1) / ROWS, P.lda);
     dim3 block(ROWS * PF * Q / 8);
     if (P.sign == FWD) launch_k<row_c2c<PF, Q, ROWS, true, TI, TO>>(grid, block, 0, s, P);
     else launch_k<row_c2c<PF, Q, ROWS, false, TI, TO>>(grid, block, 0, s, P);

@@ -48,8 +48,8 @@ struct smooth_col {
         int ja = tile * tx + c;
         const bool live = ja < P.na;
         if (!live) ja = P.na - 1;   // dead columns read the last one and store nothing
-        const C2<TI>* src = reinterpret_cast<const C2<TI>*>(P.src) + (long long)ja * P.src_s[P.fa] + (long long)jb * P.src_s[P.fb];
-        C2<TO>* dst = reinterpret_cast<C2<TO>*>(P.dst) + (long long)ja * P.dst_s[P.fa] + (long long)jb * P.dst_s[P.fb];
+        const C2<TI>* src = reinterpret_cast<const C2<TI>*>(P.from<TI>(blk.y)) + (long long)ja * P.src_s[P.fa] + (long long)jb * P.src_s[P.fb];
+        C2<TO>* dst = reinterpret_cast<C2<TO>*>(P.to<TO>(blk.y)) + (long long)ja * P.dst_s[P.fa] + (long long)jb * P.dst_s[P.fb];
         const long long sd = P.src_s[P.d], dd = P.dst_s[P.d];
         const bool inv = P.sign > 0;
         const C2<double>* tw = reinterpret_cast<const C2<double>*>(P.tw);
@@ -288,7 +288,7 @@ bool smooth_col_tile(PassDesc& P, int n) {
 }
 void launch_smooth_col(const PassDesc& P, hipStream_t s) {
     const int ntile = (P.na + P.ppb - 1) / P.ppb;
-    launch_io<smooth_col>(P, dim3(ntile * (P.n1 * P.n2 / P.na)), dim3(P.ppb * P.sm.T), (size_t)P.ppb * P.sm.M * 2 * sizeof(double), s);
+    launch_io<smooth_col>(P, dim3(ntile * (P.n1 * P.n2 / P.na), P.lda), dim3(P.ppb * P.sm.T), (size_t)P.ppb * P.sm.M * 2 * sizeof(double), s);
 }
 
 // about 128 threads a block of contiguous pencils (64: 48, 128: 36, 256: 37, 512: 45 us a pass of 200 reals),
@@ -308,8 +308,8 @@ void launch_smooth_pen(const PassDesc& P, bool col, hipStream_t s) {
     const int npen = P.n1 * P.n2;
     const size_t lds = pen_lds(P, col, P.ppb);
     const dim3 block(P.ppb * P.sm.T);
-    if (col) launch_smooth_tile(P, dim3((P.na + P.ppb - 1) / P.ppb * (npen / P.na)), block, lds, s);
-    else launch_smooth_row(P, dim3((npen + P.ppb - 1) / P.ppb), block, lds, s);
+    if (col) launch_smooth_tile(P, dim3((P.na + P.ppb - 1) / P.ppb * (npen / P.na), P.lda), block, lds, s);
+    else launch_smooth_row(P, dim3((npen + P.ppb - 1) / P.ppb, P.lda), block, lds, s);
 }
 
 // the fused last direction: columns per block (0: no smooth kernel for this length)

@@ -51,8 +51,8 @@ struct smooth_pen {
             ja = gg % P.na;
             jb = gg / P.na;
         }
-        const TI* src = reinterpret_cast<const TI*>(P.src) + ((long long)ja * P.src_s[P.fa] + (long long)jb * P.src_s[P.fb]) * P.src_nf;
-        TO* dst = reinterpret_cast<TO*>(P.dst) + ((long long)ja * P.dst_s[P.fa] + (long long)jb * P.dst_s[P.fb]) * P.dst_nf;
+        const TI* src = P.from<TI>(blk.y) + ((long long)ja * P.src_s[P.fa] + (long long)jb * P.src_s[P.fb]) * P.src_nf;
+        TO* dst = P.to<TO>(blk.y) + ((long long)ja * P.dst_s[P.fa] + (long long)jb * P.dst_s[P.fb]) * P.dst_nf;
         const long long sd = COL ? P.src_s[P.d] * P.src_nf : P.src_nf, dd = COL ? P.dst_s[P.d] * P.dst_nf : P.dst_nf;
         C2<double>* zb = reinterpret_cast<C2<double>*>(smem) + (COL ? pen : pen * (H + H / 8 + 1));
         auto slot = [&](int e) { return COL ? e * np : e + (e >> 3); };

@@ -504,7 +504,32 @@ bool SolverImpl::smooth_pass(PassDesc& P) {
     return true;
 }
 
-void SolverImpl::run_pass(PassDesc P) {
+// One pass over every component. Where their descriptions differ by the arrays alone (always, unless a
+// vector's components have their own boundary conditions), they share one launch: the blocks of three
+// small launches leave the chip half empty at each end.
+void SolverImpl::run_passes(const DirPlan& p, bool forward, const View& src, const View& dst, const Shape& tin, const Shape& tout,
+                            int gshift, int sshift) {
+    PassDesc d[3];
+    bool same = true;
+    for (int c = 0; c < lda_; ++c) {
+        d[c] = pass_desc(p, c, forward, src, dst, tin, tout, gshift, sshift);
+        const PassDesc &a = d[0], &b = d[c];
+        same = same && a.n == b.n && a.kind == b.kind && a.si == b.si && a.so == b.so && a.post == b.post && a.M == b.M &&
+               a.fastk == b.fastk && a.sm.M == b.sm.M && a.vec == b.vec && a.nt == b.nt && a.ppb == b.ppb && a.tw == b.tw &&
+               a.aux == b.aux;
+    }
+    if (same) {
+        d[0].lda = lda_;
+        d[0].src_c = src.sc;
+        d[0].dst_c = dst.sc;
+        run_pass(d[0]);
+        return;
+    }
+    SameStage stage;   // the components' launches are independent
+    for (int c = 0; c < lda_; ++c) run_pass(d[c]);
+}
+
+void SolverImpl::run_pass(const PassDesc& P) {
     if (P.sm.M > 0) {
         if (P.fastk == 5) launch_smooth_col(P, stream_);
         else launch_smooth_pen(P, P.fastk == 2 || P.fastk == 4, stream_);
@@ -796,8 +821,7 @@ void SolverImpl::forward_passes(const View& uin, void* spec) {
         const DirPlan& p = fwd_[ip];
         const View src = (ip == 0) ? uin : dense_view(dstage_[ip - 1], stage_[ip - 1], ses_);
         const View dst = dense_view(ip == ndim_ - 1 ? spec : dstage_[ip], stage_[ip], ses_);
-        SameStage same;   // the components' launches are independent
-        for (int c = 0; c < lda_; ++c) run_pass(pass_desc(p, c, true, src, dst, hat_[ip], stage_[ip], p.fieldstart, 0));
+        run_passes(p, true, src, dst, hat_[ip], stage_[ip], p.fieldstart, 0);
     }
 }
 
@@ -835,9 +859,7 @@ void SolverImpl::backward_passes(const void* spec, const View& uout, bool diff) 
         const DirPlan& p = back[ip];
         const View src = dense_view(ip == ndim_ - 1 ? const_cast<void*>(spec) : dstage_[ip], stage_[ip], ses_);
         const View dst = (ip == 0) ? uout : dense_view(dstage_[ip - 1], stage_[ip - 1], ses_);
-        SameStage same;
-        for (int c = 0; c < lda_; ++c)
-            run_pass(pass_desc(p, c, false, src, dst, stage_[ip], hat_[ip], 0, fwd_[ip].fieldstart));
+        run_passes(p, false, src, dst, stage_[ip], hat_[ip], 0, fwd_[ip].fieldstart);
     }
 }
 
@@ -849,8 +871,7 @@ void SolverImpl::solve_generic(double* field, const double* rhs, int type) {
             const DirPlan& p = fwd_[ip];
             const View src = (ip == 0) ? uin : dense_view(dstage_[ip - 1], stage_[ip - 1], ses_);
             const View dst = dense_view(dstage_[ip], stage_[ip], ses_);
-            SameStage same;
-            for (int c = 0; c < lda_; ++c) run_pass(pass_desc(p, c, true, src, dst, hat_[ip], stage_[ip], p.fieldstart, 0));
+            run_passes(p, true, src, dst, hat_[ip], stage_[ip], p.fieldstart, 0);
         }
         pmark("fftw forward");
         hybrid_z(hybrid_, dstage_[ndim_ - 2], type, stream_);
@@ -859,9 +880,7 @@ void SolverImpl::solve_generic(double* field, const double* rhs, int type) {
             const DirPlan& p = type != 0 ? bwdd_[ip] : bwd_[ip];
             const View src = dense_view(dstage_[ip], stage_[ip], ses_);
             const View dst = (ip == 0) ? uout : dense_view(dstage_[ip - 1], stage_[ip - 1], ses_);
-            SameStage same;
-            for (int c = 0; c < lda_; ++c)
-                run_pass(pass_desc(p, c, false, src, dst, stage_[ip], hat_[ip], 0, fwd_[ip].fieldstart));
+            run_passes(p, false, src, dst, stage_[ip], hat_[ip], 0, fwd_[ip].fieldstart);
         }
         pmark("fftw backward");
         return;

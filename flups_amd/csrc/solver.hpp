@@ -111,7 +111,9 @@ class SolverImpl {
     PassDesc pass_desc(const DirPlan& p, int comp, bool forward, const View& src, const View& dst, const Shape& tin,
                        const Shape& tout, int gshift, int sshift);
     bool smooth_pass(PassDesc& P);
-    void run_pass(PassDesc P);
+    void run_passes(const DirPlan& p, bool forward, const View& src, const View& dst, const Shape& tin, const Shape& tout, int gshift,
+                    int sshift);
+    void run_pass(const PassDesc& P);
     void fill_green_args(GreenArgs& A, const double hfact[3], const double kfact[3], const double koffset[3],
                          const double symstart[3], double length, int nunb);
     View user_view(double* p) const;
