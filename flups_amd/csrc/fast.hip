@@ -128,29 +128,25 @@ struct col_fft {
 // after the first one is stored.
 // HALF: nin = nout = M/2 (unbounded direction): only four rows per thread are
 // loaded and stored, the zero half is pruned from the first forward stage.
-// PF = 3: M = 3 Q (the general path's fused last direction), 8 PF values per thread through
-// column_fft_pq, no HALF pruning.
 // S: storage of the field and of G (R, or float with R = double: the general path's FP32 solves,
 // FP32 stage arrays with FP64 arithmetic)
-template <typename R, int M, int TX, int SCHED, bool HALF, int PF = 1, typename S = R>
+template <typename R, int M, int TX, int SCHED, bool HALF, typename S = R>
 struct z_fused {
     using Args = ColArgs;
-    static constexpr int NT = TX * M / (8 * PF);
-    // the mixed-radix columns: at most 256 registers per lane; the zero-padded FP32 columns up to
-    // 512 with the LDS twiddles (68 registers uncapped): 64, eight waves per SIMD, at most 16 bytes
+    static constexpr int NT = TX * M / 8;
+    // the zero-padded FP32 columns up to 512 with the LDS twiddles (68 registers uncapped): 64, eight waves per SIMD, at most 16 bytes
     // spilled (256^3: 2278 against 2254 solves/s uncapped); the other FP32 variants would spill
     // up to 80 bytes under the cap and are left uncapped
-    static constexpr int kWaves = PF == 3 ? 2 : (sizeof(R) == 4 && PF == 1 && HALF && SCHED != 1 && M <= 512 ? 8 : 0);
+    static constexpr int kWaves = sizeof(R) == 4 && HALF && SCHED != 1 && M <= 512 ? 8 : 0;
     static __device__ __forceinline__ void run(const ColArgs& a, Blk bk) {
         // SCHED 0: G loaded with the first set, second set loaded after the first is stored;
         //       1: both sets prefetched up front; 2: G loaded just before each multiply.
-        static_assert(PF == 1 || !HALF, "the zero-padded half is pruned for powers of two only");
         __shared__ C2<R> lds[M * TX];
         // FP32 (bound by its VALU instructions): the twiddle table copied to LDS, seven LDS reads
         // per radix-8 stage instead of three loads and four complex products
-        constexpr bool LTW = sizeof(R) == 4 && PF == 1;
+        constexpr bool LTW = sizeof(R) == 4;
         __shared__ C2<R> ltw[LTW ? M : 1];
-        constexpr int Q = M / PF, T = Q / 8, NV = 8 * PF;
+        constexpr int T = M / 8, NV = 8;
         const int c = threadIdx.x % TX;
         const int j = threadIdx.x / TX;
         const int ntx = (a.nx + TX - 1) / TX;
@@ -180,7 +176,6 @@ struct z_fused {
         const char* g = reinterpret_cast<const char*>(a.green) +
                         sizeof(S) * ((long long)y0 * a.gntx + a.x0 / TX + tile) * (M / 2 + 1) * TX;
         const C2<R>* tw = reinterpret_cast<const C2<R>*>(a.tw);
-        const C2<R>* twm = reinterpret_cast<const C2<R>*>(a.twm);
         R gv[NV];
         C2<R> v[NV], w[NV];
         auto load_g = [&]() {
@@ -207,14 +202,14 @@ struct z_fused {
             tw = ltw;
         }
         for (int s = 0; s < 2; ++s) {
-            column_fft_pq<R, PF, Q, true, TX, HALF, LTW>(v, lds + c, j, tw, twm, 1);
+            column_fft<R, M, true, TX, HALF, LTW>(v, lds + c, j, tw);
             if (SCHED == 2) load_g();
     #pragma unroll
             for (int i = 0; i < NV; ++i) {
                 v[i].x *= gv[i];
                 v[i].y *= gv[i];
             }
-            column_fft_pq<R, PF, Q, false, TX, false, LTW>(v, lds + c, j, tw, twm, 1);   // syncs before its first LDS write
+            column_fft<R, M, false, TX, false, LTW>(v, lds + c, j, tw);   // syncs before its first LDS write
             char* b = s == 0 ? b0 : b1;
             if (live) {
     #pragma unroll
@@ -232,62 +227,6 @@ struct z_fused {
                     load(v, b1);
                 }
             }
-        }
-    }
-};
-
-// The general path's fused last direction for M = PF Q with PF = 5 or 7: one row per block (no
-// mirror pairing), TX columns staged in LDS, PF thread teams of Q/8 threads (fft_pq_team) for
-// the forward FFT, the multiply by normfact G and the inverse FFT; in place.
-template <int PF, int Q, int TX, typename S = double>
-struct z_team {
-    using Args = ColArgs;
-    static constexpr int NT = TX * PF * Q / 8;
-    static __device__ __forceinline__ void run(const ColArgs& a, Blk bk) {
-        constexpr int M = PF * Q, T = Q / 8, TT = M / 8;
-        __shared__ C2<double> lds[M * TX];
-        const int c = threadIdx.x % TX, tt = threadIdx.x / TX;
-        const int k1 = tt / T, j = tt % T;
-        const int ntx = (a.nx + TX - 1) / TX;
-        const int blk = a.xcd ? xcd_group(bk.x, bk.nx) : bk.x;
-        const int tile = blk % ntx, y = blk / ntx;
-        const bool live = tile * TX + c < a.nx;
-        const int cl = min(c, a.nx - 1 - tile * TX);   // lanes past nx load the last valid column
-        C2<S>* col = reinterpret_cast<C2<S>*>(a.dst) + (long long)bk.y * a.comp_src + (long long)y * a.s_other_src +
-                     (long long)tile * TX;
-        // all eight loads (clamped rows, zero selected afterwards) before the LDS writes
-        C2<double> u[8];
-    #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const int r = tt + i * TT;
-            const C2<double> x = c2d(col[(long long)min(r, a.nin - 1) * a.s_col + cl]);
-            u[i] = r < a.nin ? x : C2<double>{0.0, 0.0};
-        }
-    #pragma unroll
-        for (int i = 0; i < 8; ++i) lds[(tt + i * TT) * TX + c] = u[i];
-        __syncthreads();
-        const C2<double>* tw = reinterpret_cast<const C2<double>*>(a.tw);
-        const C2<double>* twm = reinterpret_cast<const C2<double>*>(a.twm);
-        auto load = [&](int m) -> C2<double> { return lds[m * TX + c]; };
-        C2<double> v[8];
-        fft_pq_team<double, PF, Q, true, TX>(v, lds + c, k1, j, load, tw, twm, 1);
-        const S* g = reinterpret_cast<const S*>(a.green) + ((long long)y * a.gntx + tile) * (M / 2 + 1) * TX;
-    #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const int kz = k1 + PF * (j + i * T);
-            const double gv = (double)g[min(kz, M - kz) * TX + c];
-            v[i] = {v[i].x * gv, v[i].y * gv};
-        }
-        __syncthreads();   // the forward FFT's last LDS reads are done
-    #pragma unroll
-        for (int i = 0; i < 8; ++i) lds[(k1 + PF * (j + i * T)) * TX + c] = v[i];
-        __syncthreads();
-        fft_pq_team<double, PF, Q, false, TX>(v, lds + c, k1, j, load, tw, twm, 1);
-        if (!live) return;
-    #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const int r = k1 + PF * (j + i * T);
-            if (r < a.nout) col[(long long)r * a.s_col + c] = c2t<S>(v[i]);
         }
     }
 };
@@ -735,21 +674,21 @@ void launch_col_h(const ColArgs& a, int comps, int zsched, hipStream_t st) {
         // the general path's FP32 fused last direction: full- or half-width tiles, schedule 0
         const int tx = (zsched & 4) ? TX / 2 : TX;
         dim3 grid(((a.nx + tx - 1) / tx) * (a.nopair == 1 ? a.nother : a.gmy / 2 + 1), comps);
-        if (zsched & 4) launch_k<z_fused<R, M, TX / 2, 0, HALF, 1, S>>(grid, dim3(TX / 2 * M / 8), 0, st, a);
-        else launch_k<z_fused<R, M, TX, 0, HALF, 1, S>>(grid, dim3(TX * M / 8), 0, st, a);
+        if (zsched & 4) launch_k<z_fused<R, M, TX / 2, 0, HALF, S>>(grid, dim3(TX / 2 * M / 8), 0, st, a);
+        else launch_k<z_fused<R, M, TX, 0, HALF, S>>(grid, dim3(TX * M / 8), 0, st, a);
     } else if (FUSED) {
         // z schedules: bit 0-1 = SCHED of z_fused, 4 = half-width tiles (TX/2 columns)
         const int tx = (zsched & 8) ? TX / 4 : (zsched & 4) ? TX / 2 : TX;
         dim3 grid(((a.nx + tx - 1) / tx) * (a.nopair == 1 ? a.nother : a.nopair == 2 ? 2 * (a.gmy / 2 + 1) : a.gmy / 2 + 1), comps);
         switch (zsched & 15) {
-            case 0: launch_k<z_fused<R, M, TX, 0, HALF, 1, S>>(grid, dim3(TX * M / 8), 0, st, a); break;
-            case 1: launch_k<z_fused<R, M, TX, 1, HALF, 1, S>>(grid, dim3(TX * M / 8), 0, st, a); break;
-            case 2: launch_k<z_fused<R, M, TX, 2, HALF, 1, S>>(grid, dim3(TX * M / 8), 0, st, a); break;
-            case 4: launch_k<z_fused<R, M, TX / 2, 0, HALF, 1, S>>(grid, dim3(TX / 2 * M / 8), 0, st, a); break;
-            case 5: launch_k<z_fused<R, M, TX / 2, 1, HALF, 1, S>>(grid, dim3(TX / 2 * M / 8), 0, st, a); break;
-            case 6: launch_k<z_fused<R, M, TX / 2, 2, HALF, 1, S>>(grid, dim3(TX / 2 * M / 8), 0, st, a); break;
+            case 0: launch_k<z_fused<R, M, TX, 0, HALF, S>>(grid, dim3(TX * M / 8), 0, st, a); break;
+            case 1: launch_k<z_fused<R, M, TX, 1, HALF, S>>(grid, dim3(TX * M / 8), 0, st, a); break;
+            case 2: launch_k<z_fused<R, M, TX, 2, HALF, S>>(grid, dim3(TX * M / 8), 0, st, a); break;
+            case 4: launch_k<z_fused<R, M, TX / 2, 0, HALF, S>>(grid, dim3(TX / 2 * M / 8), 0, st, a); break;
+            case 5: launch_k<z_fused<R, M, TX / 2, 1, HALF, S>>(grid, dim3(TX / 2 * M / 8), 0, st, a); break;
+            case 6: launch_k<z_fused<R, M, TX / 2, 2, HALF, S>>(grid, dim3(TX / 2 * M / 8), 0, st, a); break;
             case 8:
-                launch_k<z_fused<R, M, (TX >= 8 ? TX / 4 : 1), 0, HALF, 1, S>>(grid, dim3((TX >= 8 ? TX / 4 : 1) * M / 8), 0, st, a);
+                launch_k<z_fused<R, M, (TX >= 8 ? TX / 4 : 1), 0, HALF, S>>(grid, dim3((TX >= 8 ? TX / 4 : 1) * M / 8), 0, st, a);
                 break;
             default: fail("unknown z schedule %d", zsched);
         }
@@ -1006,12 +945,10 @@ struct HybridZ {
     double normfact = 1;
     const void* g = nullptr;     // real: the solver's spectral Green's function (not owned)
     bool f32 = false;            // FP32 stage arrays and Green's function (FP64 arithmetic)
-    int pf = 1;              // M = pf 2^k: 1, or 3 (mixed-radix column FFT, 8 pf values per thread), 5, 7 (thread
-                             // teams); 0: any other smooth length (smooth_z)
+    bool smooth = false;     // not a power of two: smooth_z
     bool pair = false, twod = false;
     void* green = nullptr;   // normfact * Re G, [y'][tile][kz'][gtx]
-    void* tw = nullptr;      // (M / pf)-point table
-    void* twm = nullptr;     // M-point table (pf 3)
+    void* tw = nullptr;      // M-point table
     int rtx = 0;             // columns per block of the fused rotational pass (0: none)
     double* sym = nullptr;   // its derivative symbols: x, y, z
     size_t dev_bytes = 0;
@@ -1100,10 +1037,11 @@ HybridZ* make_hybrid_z(SolverImpl& s) {
     }
     if (in.nf != 2 || sp.nf != 2 || in.n[0] != sp.n[0] || (nd == 3 && in.n[1] != sp.n[1])) return nullptr;
     const int M = f.n_in[0];
-    const bool p2 = pow2_in(M, 32, nd == 2 ? 2048 : 1024), p3 = M % 3 == 0 && pow2_in(M / 3, 8, 128),
-               p5 = M % 5 == 0 && pow2_in(M / 5, 8, 128), p7 = M % 7 == 0 && pow2_in(M / 7, 8, 128);
-    const int smooth_tx = p2 || p3 || p5 || p7 ? 0 : smooth_z_tile(M, f32);
-    if (!(p2 || p3 || p5 || p7 || smooth_tx) || sp.n[nd - 1] != M) return nullptr;
+    // powers of two in registers; 3, 5, 7 times one on smooth_z as well (open 160^3 389 -> 338, 224^3 1032 -> 931,
+    // 48^3 70 -> 57 us against register columns and thread teams)
+    const bool p2 = pow2_in(M, 32, nd == 2 ? 2048 : 1024);
+    const int smooth_tx = p2 ? 0 : smooth_z_tile(M, f32);
+    if (!(p2 || smooth_tx) || sp.n[nd - 1] != M) return nullptr;
     const int ny = nd == 3 ? in.n[1] : 1;
     if ((double)(M / 8) * in.n[0] * ny * 16.0 >= 4294967296.0) return nullptr;
     auto* h = new HybridZ;
@@ -1120,16 +1058,8 @@ HybridZ* make_hybrid_z(SolverImpl& s) {
     // half-width x tiles in 3-D; two columns per block in 2-D (few columns, cache-resident field)
     h->gtx = nd == 2 ? 2 : 4;
     h->twod = nd == 2;
-    h->pf = p2 ? 1 : p3 ? 3 : p5 ? 5 : p7 ? 7 : 0;
-    if (h->pf == 0) h->gtx = smooth_tx;
-    if (h->pf >= 5) {   // thread teams, one row per block: no mirror pairing, tiles by length (LDS M gtx complex:
-                        // 48 KB up to M = 384, then 4 columns: 28 / 40 / 56 KB at M = 448 / 640 / 896)
-        h->pair = false;
-        h->gtx = M <= 192 ? 16 : M <= 384 ? 8 : 4;
-    }
-    // 3 Q points: Q/8 threads per column, so wider tiles keep the blocks larger (LDS M gtx
-    // complex values, 48 KB at most)
-    if (h->pf == 3) h->gtx = nd == 2 ? (M <= 96 ? 16 : 8) : (M <= 48 ? 32 : M <= 192 ? 16 : 8);
+    h->smooth = !p2;
+    if (h->smooth) h->gtx = smooth_tx;
     const int ntx = (h->nx + h->gtx - 1) / h->gtx;
     const int gy = h->pair ? h->ny / 2 + 1 : h->ny, gz = M / 2 + 1;
     const size_t gn = (size_t)gy * ntx * gz * h->gtx;
@@ -1139,16 +1069,10 @@ HybridZ* make_hybrid_z(SolverImpl& s) {
         hipLaunchKernelGGL(compress_green, dim3(4096), dim3(256), 0, s.stream_, s.dgreen_, f32 ? nullptr : (double*)h->green,
                            f32 ? (float*)h->green : nullptr, h->nx, h->ny, M, gy, gz, h->gtx, ntx, s.normfact_);
         HIP_CHECK(hipGetLastError());
-        const auto t = twiddle_table(h->pf ? M / h->pf : M);
+        const auto t = twiddle_table(M);
         HIP_CHECK(hipMalloc(&h->tw, t.size() * sizeof(double)));
         HIP_CHECK(hipMemcpy(h->tw, t.data(), t.size() * sizeof(double), hipMemcpyHostToDevice));
         h->dev_bytes += t.size() * sizeof(double);
-        if (h->pf > 1) {
-            const auto tm = twiddle_table(M);
-            HIP_CHECK(hipMalloc(&h->twm, tm.size() * sizeof(double)));
-            HIP_CHECK(hipMemcpy(h->twm, tm.data(), tm.size() * sizeof(double), hipMemcpyHostToDevice));
-            h->dev_bytes += tm.size() * sizeof(double);
-        }
         // the rotational pass: every direction unbounded or periodic, so that each derivative is i K with
         // the same real K for the three components
         bool rot = nd == 3 && s.lda_ == 3 && s.odiff_ != NOD;
@@ -1175,7 +1099,6 @@ HybridZ* make_hybrid_z(SolverImpl& s) {
         (void)hipFree(h->sym);
         (void)hipFree(h->green);
         (void)hipFree(h->tw);
-        (void)hipFree(h->twm);
         delete h;
         throw;
     }
@@ -1188,7 +1111,6 @@ void destroy_hybrid_z(HybridZ* h) {
     if (!h) return;
     (void)hipFree(h->green);
     (void)hipFree(h->tw);
-    (void)hipFree(h->twm);
     (void)hipFree(h->twn);
     (void)hipFree(h->sym);
     delete h;
@@ -1196,63 +1118,6 @@ void destroy_hybrid_z(HybridZ* h) {
 bool hybrid_runs(const HybridZ* h, int type) { return type == 0 || h->rtx > 0; }
 size_t hybrid_device_bytes(const HybridZ* h) { return h->dev_bytes; }
 double hybrid_bytes(const HybridZ* h) { return h->bytes; }
-
-// M = 3 Q: TX columns per block (the compressed G's tile width), Q/8 threads per column
-template <int M, int TX, typename S>
-void launch_z_pf3(const ColArgs& a, int comps, hipStream_t st) {
-    dim3 grid(((a.nx + TX - 1) / TX) * (a.nopair == 1 ? a.nother : a.gmy / 2 + 1), comps);
-    launch_k<z_fused<double, M, TX, 0, false, 3, S>>(grid, dim3(TX * M / 24), 0, st, a);
-    HIP_CHECK(hipGetLastError());
-}
-template <int TX, typename S>
-void dispatch_z_pf3(int M, const ColArgs& a, int comps, hipStream_t st) {
-    switch (M) {
-        case 24: launch_z_pf3<24, TX, S>(a, comps, st); break;
-        case 48: launch_z_pf3<48, TX, S>(a, comps, st); break;
-        case 96:
-            if constexpr (TX <= 16) launch_z_pf3<96, TX, S>(a, comps, st);
-            else fail("column length %d with tiles of %d", M, TX);
-            break;
-        case 192:
-            if constexpr (TX <= 16) launch_z_pf3<192, TX, S>(a, comps, st);
-            else fail("column length %d with tiles of %d", M, TX);
-            break;
-        case 384:
-            if constexpr (TX <= 8) launch_z_pf3<384, TX, S>(a, comps, st);
-            else fail("column length %d with tiles of %d", M, TX);
-            break;
-        default: fail("unsupported column length %d", M);
-    }
-}
-
-template <int PF, int Q, typename S>
-void launch_z_team(int tx, const ColArgs& a, int comps, hipStream_t st) {
-    const int ntx = (a.nx + tx - 1) / tx;
-    dim3 grid(ntx * a.nother, comps);
-    switch (tx) {
-        case 16:
-            if constexpr (PF * Q <= 192) launch_k<z_team<PF, Q, 16, S>>(grid, dim3(16 * PF * Q / 8), 0, st, a);
-            else fail("column length %d with tiles of 16", PF * Q);
-            break;
-        case 8:
-            if constexpr (PF * Q <= 384) launch_k<z_team<PF, Q, 8, S>>(grid, dim3(8 * PF * Q / 8), 0, st, a);
-            else fail("column length %d with tiles of 8", PF * Q);
-            break;
-        default: launch_k<z_team<PF, Q, 4, S>>(grid, dim3(4 * PF * Q / 8), 0, st, a); break;
-    }
-    HIP_CHECK(hipGetLastError());
-}
-template <int PF, typename S>
-void dispatch_z_team(int M, int tx, const ColArgs& a, int comps, hipStream_t st) {
-    switch (M / PF) {
-        case 8: launch_z_team<PF, 8, S>(tx, a, comps, st); break;
-        case 16: launch_z_team<PF, 16, S>(tx, a, comps, st); break;
-        case 32: launch_z_team<PF, 32, S>(tx, a, comps, st); break;
-        case 64: launch_z_team<PF, 64, S>(tx, a, comps, st); break;
-        case 128: launch_z_team<PF, 128, S>(tx, a, comps, st); break;
-        default: fail("unsupported column length %d", M);
-    }
-}
 
 // in place on the stage array before the z transform: (nx, ny, nz) complex (real for an r2c
 // last direction), lda components; S = the storage of the stage array (float for FP32 solves)
@@ -1291,7 +1156,7 @@ void hybrid_z_t(const HybridZ* h, void* data, hipStream_t st) {
         launch_col_rz(A, st);
         return;
     }
-    if (h->pf == 0) {
+    if (h->smooth) {
         SmoothZArgs A;
         A.f32 = std::is_same<S, float>::value;
         A.d = data;
@@ -1333,20 +1198,6 @@ void hybrid_z_t(const HybridZ* h, void* data, hipStream_t st) {
     z.nopair = h->pair ? 0 : 1;
     z.x0 = 0;
     z.gntx = (h->nx + h->gtx - 1) / h->gtx;
-    z.twm = h->twm;
-    if (h->pf >= 5) {
-        if (h->pf == 5) dispatch_z_team<5, S>(h->M, h->gtx, z, h->lda, st);
-        else dispatch_z_team<7, S>(h->M, h->gtx, z, h->lda, st);
-        return;
-    }
-    if (h->pf == 3) {
-        switch (h->gtx) {
-            case 32: dispatch_z_pf3<32, S>(h->M, z, h->lda, st); break;
-            case 16: dispatch_z_pf3<16, S>(h->M, z, h->lda, st); break;
-            default: dispatch_z_pf3<8, S>(h->M, z, h->lda, st); break;
-        }
-        return;
-    }
     if (h->twod) {   // two columns per block (the tile width of the compressed G), XCD-grouped
         switch (h->M) {
             case 32: launch_col<double, 32, 2, true, true, S>(z, h->lda, 16, st); break;
@@ -1369,7 +1220,7 @@ void hybrid_z(const HybridZ* h, void* data, int type, hipStream_t st) {
         SmoothRotArgs A;
         A.d = data;
         A.g = h->green;
-        A.tw = static_cast<const double*>(h->pf > 1 ? h->twm : h->tw);
+        A.tw = static_cast<const double*>(h->tw);
         A.sym = h->sym;
         A.off[1] = h->nx;
         A.off[2] = h->nx + h->ny;

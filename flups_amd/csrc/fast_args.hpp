@@ -26,7 +26,6 @@ struct ColArgs {
     int x0;              // z_fused / z_rot: spectral x index of column 0 (slab offset, a multiple of TX)
     int gntx;            // z_fused / z_rot: x tiles of one ky' row of the compressed G
     int gtx;             // z_rot: tile width of the compressed G
-    const void* twm;     // z_fused with PF > 1: M-point twiddle table (tw is then the M/PF-point one)
     int nt;              // col_fft forward: 1 = non-temporal stores
 };
 

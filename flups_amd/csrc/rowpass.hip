@@ -68,13 +68,13 @@ bool c2c_pencil_ok(const PassDesc& P) {
 
 namespace {
 // the plan semantics the r2r pencil kernels reproduce (kinds, length, offsets, corrections)
-bool r2r_plan_fits(const PassDesc& P, bool smooth) {
+bool r2r_plan_fits(const PassDesc& P, bool smooth, int maxpf) {
     const int k = P.kind;
     const int n = P.n, h = r2r_h(k, n);
     if (P.op != OP_R2R) return false;
     const bool e00 = k == REDFT00 || k == RODFT00;
     if (!(e00 || k == REDFT10 || k == REDFT01 || k == REDFT11 || k == RODFT10 || k == RODFT01 || k == RODFT11)) return false;
-    if ((!e00 && n % 2) || !len_ok(smooth, h, 16, 1024, 7)) return false;
+    if ((!e00 && n % 2) || !len_ok(smooth, h, 16, 1024, maxpf)) return false;
     if (!(P.src_nf == 1 && P.dst_nf == 1 && P.nf_in == 1 && P.nf_out == 1 && P.r2r_stride == 1 && P.pen_in == P.pen_out &&
           P.pen_in >= n && P.pen_in <= n + 2 && P.gshift >= 0 && P.sshift >= 0))
         return false;
@@ -89,10 +89,22 @@ bool r2r_plan_fits(const PassDesc& P, bool smooth) {
 }
 }  // namespace
 
-bool row_r2r_fits(const PassDesc& P, bool smooth) { return r2r_plan_fits(P, smooth) && P.src_s[P.d] == 1 && P.dst_s[P.d] == 1; }
+// Which lengths 3, 5, 7 times a power of two run on thread teams (smooth = false) and which on the kernels of
+// smooth.hip was measured on whole solves (MI355X, FP64, us, teams -> smooth). Rows, DCT / DST-II and III:
+// 5, 7 and the short 3 on smooth (plate 224 x 128 x 128 153 -> 139, 96 x 64 x 64 60.5 -> 55.7; 192: 125 -> 127);
+// kind IV, whose pre-map pairs x[2m] with x[n-1-2m], on teams (mixed 160 x 128 x 128 75 -> 86).
+bool row_r2r_fits(const PassDesc& P, bool smooth) {
+    const bool k23 = P.kind == REDFT10 || P.kind == REDFT01 || P.kind == RODFT10 || P.kind == RODFT01;
+    int pf = 1, q = 0;
+    const int h = r2r_h(P.kind, P.n);
+    if (!smooth && k23 && split_pq(h, pf, q) && pf > 1 && (pf > 3 || h < 96)) return false;
+    return r2r_plan_fits(P, smooth, 7) && P.src_s[P.d] == 1 && P.dst_s[P.d] == 1;
+}
 
+// columns: 5 and 7 on smooth (node-centred 129 x 161 x 97 165 -> 145, channel 160^3 184 -> 171); 3 stays
+// (channel 64 x 192 x 64 74 -> 77), powers of two too (channel 256^3 452 -> 483)
 bool col_r2r_fits(const PassDesc& P, bool smooth) {
-    return r2r_plan_fits(P, smooth) && P.fa != P.d && P.src_s[P.fa] == 1 && P.dst_s[P.fa] == 1 && (P.n1 * P.n2) % P.na == 0;
+    return r2r_plan_fits(P, smooth, 3) && P.fa != P.d && P.src_s[P.fa] == 1 && P.dst_s[P.fa] == 1 && (P.n1 * P.n2) % P.na == 0;
 }
 
 // pre / post twiddles of the row r2r kernels, (H + 1) complex each, exact to rounding
@@ -140,11 +152,12 @@ bool rc_plan_fits(const PassDesc& P) {
 }
 }  // namespace
 
-bool row_rc_fits(const PassDesc& P, bool smooth) {
-    const int h = P.n / 2;
-    if (!rc_plan_fits(P) || P.src_s[P.d] != 1 || P.dst_s[P.d] != 1 || !len_ok(smooth, h, 16, 1024, 7)) return false;
-    // buffer of the pencil in LDS: at most 2H + H/4 doubles (the kernels of smooth.hip size it at the launch)
-    return smooth || (P.pen_in * P.nf_in <= 2 * h + h / 4 && P.pen_out * P.nf_out <= 2 * h + h / 4);
+// contiguous r2c / c2r of a smooth length. Powers of two too: the pencils straight between HBM and the first /
+// last stage beat the copy through LDS of the earlier register kernel (periodic 160^3 131 -> 111,
+// channel 256^3 452 -> 418, 2-D 1024^2 73 -> 67 us)
+bool row_rc_fits(const PassDesc& P) {
+    SmoothPlan p;
+    return rc_plan_fits(P) && P.src_s[P.d] == 1 && P.dst_s[P.d] == 1 && smooth_plan(P.n / 2, p);
 }
 
 // strided r2c / c2r of a smooth length, neighbouring pencils along a unit-stride dimension
@@ -157,7 +170,9 @@ bool col_rc_fits(const PassDesc& P) {
 
 bool col_real_fits(const PassDesc& P) {
     const int n = P.n;
-    if (!(P.op == OP_R2C || P.op == OP_C2R) || !fft_len_ok(n, 32, 1024, 5)) return false;   // 8 PF values per thread
+    // 8 PF values per thread; 5 times a power of two on smooth.hip (mixed 160^3 154 -> 133 us), 3 here (mixed
+    // 96^3 62.5 against 64.4)
+    if (!(P.op == OP_R2C || P.op == OP_C2R) || !fft_len_ok(n, 32, 1024, 3)) return false;
     const bool fwd = P.op == OP_R2C;
     const int d = P.d, fa = P.fa;
     if (fa == d || P.src_s[fa] != 1 || P.dst_s[fa] != 1) return false;
@@ -181,6 +196,9 @@ bool col_real_fits(const PassDesc& P) {
 bool col_c2c_fits(const PassDesc& P, bool smooth) {
     const int n = P.n;
     if (P.op != OP_C2C || !len_ok(smooth, n, 32, 2048, 7) || P.M != n) return false;
+    // 3, 5, 7 times a power of two above 256: smooth.hip (open 160 x 192 x 128 301 -> 264 us, 64 x 320 x 64 123 -> 109;
+    // below, its blocks of 64 threads and one radix above 10 lose 1 to 4 us of 60 to 80)
+    if (!smooth && n > 256 && (n & (n - 1))) return false;
     const int d = P.d, fa = P.fa;
     if (fa == d || P.src_s[fa] != 1 || P.dst_s[fa] != 1 || (P.n1 * P.n2) % P.na != 0) return false;
     if (!(P.nf_in == 2 && P.nf_out == 2 && P.src_nf == 2 && P.dst_nf == 2 && c2c_pencil_ok(P))) return false;
@@ -200,7 +218,6 @@ bool row_rz_len_ok(int M) { return M % 2 == 0 && fft_len_ok(M / 2, 16, 1024, 7);
 
 void launch_row_r2r(const PassDesc& P, hipStream_t s) { rowpass_io(RP_ROW_R2R, P, s); }
 void launch_col_r2r(const PassDesc& P, hipStream_t s) { rowpass_io(RP_COL_R2R, P, s); }
-void launch_row_rc(const PassDesc& P, hipStream_t s) { rowpass_io(RP_ROW_RC, P, s); }
 void launch_col_real(const PassDesc& P, hipStream_t s) { rowpass_io(RP_COL_REAL, P, s); }
 void launch_col_c2c(const PassDesc& P, hipStream_t s) { rowpass_io(RP_COL_C2C, P, s); }
 void launch_row_c2c(const PassDesc& P, hipStream_t s) { rowpass_io(RP_ROW_C2C, P, s); }

@@ -49,19 +49,13 @@
 // strided direction, TX neighbouring pencils per block, with the zero padding of the gather
 // and the truncation of the scatter (the second and third transforms of unbounded and
 // periodic directions in the general path). col_c2c_team: the same for M = 5 or 7 times a
-// power of two, the columns staged in LDS first.
+// power of two up to 256, the columns staged in LDS first.
 //
 // row_c2c: c2c of length M (in [16, 1024]) along a contiguous pencil (x after an r2c
 // direction), staged in LDS, PF teams of M/(8 PF) threads.
 //
 // col_rz: the general path's last direction when it is an r2c one, with the multiply: r2c,
 // normfact G, c2r of paired real columns in one in-place launch; row_rz: the same along x.
-//
-// row_rc: r2c / c2r of even length n = 2H (H in [16, 1024]) along a
-// contiguous pencil through the packed complex FFT of length H: z[m] = x[2m] + i x[2m+1],
-// X[k] = (Z[k] + conj Z[H-k])/2 + e^{-2 pi i k/n} (Z[k] - conj Z[H-k])/(2i), k <= H; the
-// inverse Z[k] = (X[k] + conj X[H-k]) + i e^{2 pi i k/n} (X[k] - conj X[H-k]), x[2m] + i x[2m+1]
-// = IFFT_H(Z) (the imaginary parts of X[0] and X[H] ignored).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -310,113 +304,6 @@ struct pen_r2r {
     }
 };
 
-// H = PF Q: PF = 1 (a power of two) or 3, 5, 7 (PF teams of Q/8 threads, fft_pq_team);
-// H/8 threads per row either way
-template <int PF, int Q, int ROWS, bool FWD, typename TI, typename TO>
-struct row_rc {
-    using Args = PassDesc;
-    static constexpr int NT = ROWS * PF * Q / 8;
-    static __device__ __forceinline__ void run(const PassDesc& P, Blk blk) {
-        constexpr int H = PF * Q, T = Q / 8, TT = H / 8, HP = H + H / 8;
-        __shared__ C2<double> lds[HP * ROWS];
-        const int rl = threadIdx.x / TT, tt = threadIdx.x % TT;
-        const int k1 = tt / T, j = tt % T;   // team and thread in the team
-        const int g = blk.x * ROWS + rl;
-        const bool live = g < P.n1 * P.n2;
-        const int gg = live ? g : 0;   // dead rows read pencil 0 and store nothing
-        const int ja = gg % P.na, jb = gg / P.na;
-        const TI* src = P.from<TI>(blk.y) + (long long)ja * P.src_s[P.fa] * P.src_nf + (long long)jb * P.src_s[P.fb] * P.src_nf;
-        TO* dst = P.to<TO>(blk.y) + (long long)ja * P.dst_s[P.fa] * P.dst_nf + (long long)jb * P.dst_s[P.fb] * P.dst_nf;
-        C2<double>* row = lds + rl * HP;
-        double* rd = reinterpret_cast<double*>(row);
-        const C2<double>* tw = reinterpret_cast<const C2<double>*>(P.tw);    // Q-point table
-        const C2<double>* twn = reinterpret_cast<const C2<double>*>(P.aux);  // n-point table
-        // 1. gather: the pencil's doubles (reals for r2c, interleaved complex for c2r)
-        const int nfi = P.nf_in, len = P.pen_in * nfi;
-        const int last = max(P.src_nd - 1, 0);
-        staged_gather<8>(tt, TT, len, [&](int q) {
-            const int k = q / nfi, ks = k - P.gshift;
-            const double x = (double)src[(long long)min(max(ks, 0), last) * nfi + (q - k * nfi)];
-            return (ks >= 0 && ks < P.src_nd) ? x : 0.0;
-        }, [&](int q, double x) { rd[q] = x; });
-        __syncthreads();
-        // element m of the packed complex sequence: z[m] = x[2m] + i x[2m+1] (r2c), or built from
-        // X[m] and X[H-m] (c2r)
-        auto c2r_z = [&](int m) -> C2<double> {
-            C2<double> a = {rd[2 * m], rd[2 * m + 1]}, b = {rd[2 * (H - m)], rd[2 * (H - m) + 1]};
-            if (m == 0) {   // DC and Nyquist are real
-                a.y = 0.0;
-                b.y = 0.0;
-            }
-            const C2<double> bc = cconj(b);
-            const C2<double> e = cadd(a, bc), f = csub(a, bc);
-            const C2<double> t = cmul(cconj(twn[m]), f);   // e^{+2 pi i m/n} (a - conj b)
-            return {e.x - t.y, e.y + t.x};
-        };
-        // mixed radix (PF > 1) reads every input PF times: build z in the row first, the pairs
-        // (m, H - m) by one thread, so that the transform's loads are plain LDS reads (inlined into
-        // its PF-fold unrolled loads, the construction held several hundred registers live)
-        constexpr bool PRE = !FWD && PF > 1;
-        if constexpr (PRE) {
-            for (int m = tt; m <= H / 2; m += TT) {
-                const C2<double> zm = c2r_z(m);
-                const C2<double> zh = (m > 0 && 2 * m != H) ? c2r_z(H - m) : C2<double>{0, 0};
-                row[m] = zm;
-                if (m > 0 && 2 * m != H) row[H - m] = zh;
-            }
-            __syncthreads();
-        }
-        auto load = [&](int m) -> C2<double> {
-            if (FWD || PRE) return {rd[2 * m], rd[2 * m + 1]};
-            return c2r_z(m);
-        };
-        C2<double> v[8];
-        fft_pq_team<double, PF, Q, FWD, 0>(v, row, k1, j, load, tw, twn, 2);   // w_H^e = twn[2 e]
-        __syncthreads();
-        const int nfo = P.nf_out, plen = P.pen_out;
-        // v[i] = Z[k1 + PF (j + i T)]
-    #pragma unroll
-        for (int i = 0; i < 8; ++i) row[k1 + PF * (j + i * T)] = v[i];
-        if (FWD) {
-            // X[k], k <= H, into the row as complex values
-            __syncthreads();
-            C2<double> XH = {0, 0};
-    #pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                const int k = tt + i * TT;
-                const C2<double> zk = row[k], zc = cconj(row[k == 0 ? 0 : H - k]);
-                const C2<double> e = {0.5 * (zk.x + zc.x), 0.5 * (zk.y + zc.y)};
-                const C2<double> df = {0.5 * (zk.x - zc.x), 0.5 * (zk.y - zc.y)};
-                v[i] = cadd(e, cmul(twn[k], C2<double>{df.y, -df.x}));
-            }
-            if (tt == 0) {
-                const C2<double> z0 = row[0];
-                XH = {z0.x - z0.y, 0.0};
-            }
-            __syncthreads();
-    #pragma unroll
-            for (int i = 0; i < 8; ++i) row[tt + i * TT] = v[i];
-            if (tt == 0) row[H] = XH;
-            // positions past H + 1 complex values keep nothing (zero)
-            for (int q = H + 1 + tt; q < plen; q += TT) row[q] = {0.0, 0.0};
-            // periodic node-centred direction: the first value again at the end (n_out - 1)
-            if ((P.post & POST_PERIOD) && tt == 0) row[P.n_out_plan - 1] = v[0];
-        } else {
-            // x[2m] = Re z[m], x[2m+1] = Im z[m] (written above)
-            for (int q = 2 * H + tt; q < plen; q += TT) rd[q] = 0.0;
-            if ((P.post & POST_PERIOD) && tt == 0) rd[2 * H] = v[0].x;   // x[n] = x[0]
-        }
-        __syncthreads();
-        if (!live) return;
-        // 2. scatter (truncation), element k of the destination = pencil position k + sshift
-        const int dn = P.dst_nd;
-        for (int q = tt; q < dn * nfo; q += TT) {
-            const int k = q / nfo, p = k + P.sshift;
-            if (p < plen) dst[(long long)k * nfo + (q - k * nfo)] = (TO)rd[p * nfo + (q - k * nfo)];
-        }
-    }
-};
-
 // M = PF Q: PF = 1 (a power of two) or 3, 5 (8 PF values per thread, column_fft_pq)
 template <int PF, int Q, int TX, bool FWD, typename TI, typename TO>
 struct col_real {
@@ -589,7 +476,7 @@ struct col_rz {
 // The general path's last direction when it is an r2c along x (every other direction real-
 // to-real): r2c of each row (length n = 2H, rows zero-padded from nin), X[k] normfact G[k]
 // (G real, one row of the spectral layout per field row), c2r, the first nin values stored,
-// all in LDS, in place. PF teams of Q/8 threads as row_rc.
+// all in LDS, in place. H = PF Q: PF = 1 or PF teams of Q/8 threads (fft_pq_team).
 template <int PF, int Q, int ROWS, typename S>
 struct row_rz {
     using Args = RzArgs;
@@ -653,7 +540,7 @@ struct row_rz {
             const C2<double> t = cmul(cconj(twn[m]), f);
             return {e.x - t.y, e.y + t.x};
         };
-        // mixed radix: Z built in the row first (as in row_rc's c2r), the transform reads it plainly
+        // mixed radix: Z built in the row first (as in a c2r), the transform reads it plainly
         constexpr bool PRE = PF > 1;
         if constexpr (PRE) {
             for (int m = tt; m <= H / 2; m += TT) {
@@ -825,12 +712,18 @@ void launch_pen_h(const PassDesc& P, hipStream_t s) {
     const int nb = COL ? ((P.na + R - 1) / R) * (npen / P.na) : (npen + R - 1) / R;
     dim3 grid(nb, P.lda);
     dim3 block(R * PF * Q / 8);
+    // DCT / DST-II and III of 5 and 7 times a power of two: smooth.hip
+    if constexpr (PF <= 3) {
+        switch (P.kind) {
+            case REDFT10: launch_k<pen_r2r<PF, Q, R, REDFT10, COL, TI, TO>>(grid, block, 0, s, P); return;
+            case REDFT01: launch_k<pen_r2r<PF, Q, R, REDFT01, COL, TI, TO>>(grid, block, 0, s, P); return;
+            case RODFT10: launch_k<pen_r2r<PF, Q, R, RODFT10, COL, TI, TO>>(grid, block, 0, s, P); return;
+            case RODFT01: launch_k<pen_r2r<PF, Q, R, RODFT01, COL, TI, TO>>(grid, block, 0, s, P); return;
+            default: break;
+        }
+    }
     switch (P.kind) {
-        case REDFT10: launch_k<pen_r2r<PF, Q, R, REDFT10, COL, TI, TO>>(grid, block, 0, s, P); break;
-        case REDFT01: launch_k<pen_r2r<PF, Q, R, REDFT01, COL, TI, TO>>(grid, block, 0, s, P); break;
         case REDFT11: launch_k<pen_r2r<PF, Q, R, REDFT11, COL, TI, TO>>(grid, block, 0, s, P); break;
-        case RODFT10: launch_k<pen_r2r<PF, Q, R, RODFT10, COL, TI, TO>>(grid, block, 0, s, P); break;
-        case RODFT01: launch_k<pen_r2r<PF, Q, R, RODFT01, COL, TI, TO>>(grid, block, 0, s, P); break;
         case RODFT11: launch_k<pen_r2r<PF, Q, R, RODFT11, COL, TI, TO>>(grid, block, 0, s, P); break;
         case REDFT00: launch_k<pen_r2r<PF, Q, R, REDFT00, COL, TI, TO>>(grid, block, 0, s, P); break;
         case RODFT00: launch_k<pen_r2r<PF, Q, R, RODFT00, COL, TI, TO>>(grid, block, 0, s, P); break;
@@ -852,26 +745,6 @@ void launch_pen_pf(int q, const PassDesc& P, hipStream_t s) {
     }
 }
 
-template <int PF, int Q, int ROWS, typename TI, typename TO>
-void launch_row_rc_h(const PassDesc& P, hipStream_t s) {
-    dim3 grid((P.n1 * P.n2 + ROWS - 1) / ROWS, P.lda);
-    dim3 block(ROWS * PF * Q / 8);
-    if (P.op == OP_R2C) launch_k<row_rc<PF, Q, ROWS, true, TI, TO>>(grid, block, 0, s, P);
-    else launch_k<row_rc<PF, Q, ROWS, false, TI, TO>>(grid, block, 0, s, P);
-}
-// H = PF Q, 3 <= PF <= 7: about 256 threads (2048 / H rows) and 36 KB of LDS per block
-template <int PF, typename TI, typename TO>
-void launch_row_rc_pf(int q, const PassDesc& P, hipStream_t s) {
-    switch (q) {
-        case 8: launch_row_rc_h<PF, 8, 2048 / (PF * 8), TI, TO>(P, s); break;
-        case 16: launch_row_rc_h<PF, 16, 2048 / (PF * 16), TI, TO>(P, s); break;
-        case 32: launch_row_rc_h<PF, 32, 2048 / (PF * 32), TI, TO>(P, s); break;
-        case 64: launch_row_rc_h<PF, 64, 2048 / (PF * 64), TI, TO>(P, s); break;
-        case 128: launch_row_rc_h<PF, 128, 2048 / (PF * 128), TI, TO>(P, s); break;
-        default: fail("row rc: length %d", P.n);
-    }
-}
-
 template <int PF, int Q, int TX, typename TI, typename TO>
 void launch_col_real_m(const PassDesc& P, hipStream_t s) {
     const int npair = (P.na + 1) / 2;
@@ -881,10 +754,10 @@ void launch_col_real_m(const PassDesc& P, hipStream_t s) {
     if (P.op == OP_R2C) launch_k<col_real<PF, Q, TX, true, TI, TO>>(grid, dim3(TX * Q / 8), 0, s, P);
     else launch_k<col_real<PF, Q, TX, false, TI, TO>>(grid, dim3(TX * Q / 8), 0, s, P);
 }
-// mixed radix: TX Q = 1024 (PF 3) or 512 (PF 5), LDS about 48 / 40 KB
+// mixed radix, PF = 3: TX Q = 1024, LDS about 48 KB
 template <int PF, typename TI, typename TO>
 void launch_col_real_pf(int q, const PassDesc& P, hipStream_t s) {
-    constexpr int TQ = PF == 3 ? 1024 : 512;
+    constexpr int TQ = 1024;
     switch (q) {
         case 8: launch_col_real_m<PF, 8, TQ / 8, TI, TO>(P, s); break;
         case 16: launch_col_real_m<PF, 16, TQ / 16, TI, TO>(P, s); break;
@@ -937,32 +810,28 @@ void launch_row_c2c_pf(int q, const PassDesc& P, hipStream_t s) {
         default: fail("row c2c: length %d", P.n);
     }
 }
-// thread teams: TX M <= 4096 (64 KB of LDS), TX >= 4
+// thread teams, M <= 256
 template <int PF, typename TI, typename TO>
 void launch_col_c2c_team_pf(int q, const PassDesc& P, hipStream_t s) {
     switch (q) {
         case 8: launch_col_c2c_t<PF, 8, 16, TI, TO>(P, s); break;
         case 16: launch_col_c2c_t<PF, 16, 16, TI, TO>(P, s); break;
-        case 32: launch_col_c2c_t<PF, 32, (PF * 32 <= 128 ? 16 : 8), TI, TO>(P, s); break;
-        case 64: launch_col_c2c_t<PF, 64, (PF * 64 <= 256 ? 16 : PF * 64 <= 512 ? 8 : 4), TI, TO>(P, s); break;
-        case 128: launch_col_c2c_t<PF, 128, (PF * 128 <= 512 ? 8 : 4), TI, TO>(P, s); break;
+        case 32: launch_col_c2c_t<PF, 32, 8, TI, TO>(P, s); break;
         default: fail("column c2c: length %d", P.n);
     }
 }
-// mixed radix, 8 PF values per thread: TX Q = 1024 (PF 3) or 512, LDS 48 / 40 KB
+// mixed radix, 8 PF values per thread, PF = 3, M <= 256: TX Q = 1024, LDS 48 KB
 template <int PF, typename TI, typename TO>
 void launch_col_c2c_pf(int q, const PassDesc& P, hipStream_t s) {
-    constexpr int TQ = PF == 3 ? 1024 : 512;
+    constexpr int TQ = 1024;
     switch (q) {
         case 8: launch_col_c2c_m<PF, 8, TQ / 8, TI, TO>(P, s); break;
         case 16: launch_col_c2c_m<PF, 16, TQ / 16, TI, TO>(P, s); break;
         case 32: launch_col_c2c_m<PF, 32, TQ / 32, TI, TO>(P, s); break;
         case 64: launch_col_c2c_m<PF, 64, TQ / 64, TI, TO>(P, s); break;
-        case 128: launch_col_c2c_m<PF, 128, TQ / 128, TI, TO>(P, s); break;
         default: fail("column c2c: length %d", P.n);
     }
 }
-
 
 template <int M, int TX, typename S>
 void launch_col_rz_m(const RzArgs& A, hipStream_t s) {
@@ -989,36 +858,12 @@ void launch_row_rz_pf(int q, const RzArgs& A, hipStream_t s) {
 }
 
 template <typename TI, typename TO>
-void launch_row_rc_t(const PassDesc& P, hipStream_t s) {
-    int pf = 1, q = 0;
-    split_pq(P.n / 2, pf, q);
-    if (pf != 1) {
-        if (pf == 3) launch_row_rc_pf<3, TI, TO>(q, P, s);
-        else if (pf == 5) launch_row_rc_pf<5, TI, TO>(q, P, s);
-        else launch_row_rc_pf<7, TI, TO>(q, P, s);
-        HIP_CHECK(hipGetLastError());
-        return;
-    }
-    switch (P.n / 2) {
-        case 16: launch_row_rc_h<1, 16, 128, TI, TO>(P, s); break;
-        case 32: launch_row_rc_h<1, 32, 64, TI, TO>(P, s); break;
-        case 64: launch_row_rc_h<1, 64, 32, TI, TO>(P, s); break;
-        case 128: launch_row_rc_h<1, 128, 16, TI, TO>(P, s); break;
-        case 256: launch_row_rc_h<1, 256, 8, TI, TO>(P, s); break;
-        case 512: launch_row_rc_h<1, 512, 4, TI, TO>(P, s); break;
-        case 1024: launch_row_rc_h<1, 1024, 2, TI, TO>(P, s); break;
-        default: fail("row rc: length %d", P.n);
-    }
-    HIP_CHECK(hipGetLastError());
-}
-
-template <typename TI, typename TO>
 void launch_col_real_t(const PassDesc& P, hipStream_t s) {
     int pf = 1, q = 0;
     split_pq(P.n, pf, q);
     if (pf != 1) {
-        if (pf == 3) launch_col_real_pf<3, TI, TO>(q, P, s);
-        else launch_col_real_pf<5, TI, TO>(q, P, s);
+        FLUPS_REQUIRE(pf == 3, "col real: length %d", P.n);
+        launch_col_real_pf<3, TI, TO>(q, P, s);
         HIP_CHECK(hipGetLastError());
         return;
     }
@@ -1155,9 +1000,8 @@ void launch_col_r2r_t(const PassDesc& P, hipStream_t s) {
     int pf = 1, q = 0;
     split_pq(h, pf, q);
     if (pf != 1) {
-        if (pf == 3) launch_pen_pf<3, true, TI, TO>(q, P, s);
-        else if (pf == 5) launch_pen_pf<5, true, TI, TO>(q, P, s);
-        else launch_pen_pf<7, true, TI, TO>(q, P, s);
+        FLUPS_REQUIRE(pf == 3, "column r2r: length %d", P.n);
+        launch_pen_pf<3, true, TI, TO>(q, P, s);
         HIP_CHECK(hipGetLastError());
         return;
     }
@@ -1177,7 +1021,7 @@ void launch_col_r2r_t(const PassDesc& P, hipStream_t s) {
 }  // namespace
 
 // the passes of one (TI, TO) storage combination, compiled in its own translation unit
-enum RowpassKernel { RP_ROW_R2R, RP_COL_R2R, RP_ROW_RC, RP_COL_REAL, RP_COL_C2C, RP_ROW_C2C };
+enum RowpassKernel { RP_ROW_R2R, RP_COL_R2R, RP_COL_REAL, RP_COL_C2C, RP_ROW_C2C };
 void rowpass_dd(int which, const PassDesc& P, hipStream_t s);
 void rowpass_df(int which, const PassDesc& P, hipStream_t s);
 void rowpass_ff(int which, const PassDesc& P, hipStream_t s);
@@ -1190,7 +1034,6 @@ void rz_f(int row, const RzArgs& A, hipStream_t s);
         switch (which) {                                                \
             case RP_ROW_R2R: launch_row_r2r_t<TI, TO>(P, s); break;     \
             case RP_COL_R2R: launch_col_r2r_t<TI, TO>(P, s); break;     \
-            case RP_ROW_RC: launch_row_rc_t<TI, TO>(P, s); break;       \
             case RP_COL_REAL: launch_col_real_t<TI, TO>(P, s); break;   \
             case RP_COL_C2C: launch_col_c2c_t<TI, TO>(P, s); break;     \
             default: launch_row_c2c_t<TI, TO>(P, s); break;             \

@@ -1,6 +1,7 @@
-// Pass kernels of the general path for the lengths with factors 2, 3, 5, 7 that the register
-// kernels of rowpass.hip do not have (9, 15, 25, ... times a power of two: 100, 120, 144, 180, 200,
-// 240, 300, ...), on the run-time mixed-radix FFT of smooth_fft.hpp:
+// Pass kernels of the general path for lengths with factors 2, 3, 5, 7 on the run-time mixed-radix FFT of
+// smooth_fft.hpp: every length that the register kernels of rowpass.hip do not have (9, 15, 25, ... times a
+// power of two: 100, 120, 144, 180, 200, 240, 300, ...), and of the others the passes that they run faster
+// (contiguous r2c / c2r of every length; the rules stand at the fit tests in rowpass.hip):
 //   smooth_col   c2c along a strided direction, values straight between HBM and the first / last
 //                stage's registers;
 //   smooth_z     the last direction fused with the multiply: forward c2c, normfact G, inverse c2c;
@@ -226,6 +227,7 @@ static bool search_plan(int M, SmoothPlan& p) {
     std::vector<int> cur, best;
     auto search = [&](auto&& self, int m, int lo) -> void {
         if (m == 1) {
+            if (cur.size() < 2) return;
             const bool low = cur.back() <= 10, blow = !best.empty() && best.back() <= 10;
             if (best.empty() || cur.size() < best.size() ||
                 (cur.size() == best.size() && (low != blow ? low : cur[0] > best[0])))
@@ -241,7 +243,7 @@ static bool search_plan(int M, SmoothPlan& p) {
             }
     };
     search(search, M, 0);
-    if (best.size() < 2) return false;
+    if (best.empty()) return false;
     p = SmoothPlan();
     p.M = M;
     p.nst = (int)best.size();
@@ -267,7 +269,7 @@ static bool search_plan(int M, SmoothPlan& p) {
 }
 // every pass of every solve asks: the answers (a function of M alone, at most 2031 of them) are kept
 bool smooth_plan(int M, SmoothPlan& p) {
-    if (M < 18 || M > 2048) return false;
+    if (M < 16 || M > 2048) return false;
     static std::mutex mu;
     static std::map<int, SmoothPlan> known;   // M = 0: no plan
     std::lock_guard<std::mutex> lk(mu);

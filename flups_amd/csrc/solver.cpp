@@ -28,9 +28,8 @@ void launch_generic(const PassDesc& P, hipStream_t s);
 bool row_r2r_fits(const PassDesc& P, bool smooth = false);
 bool col_real_fits(const PassDesc& P);
 void launch_col_real(const PassDesc& P, hipStream_t s);
-bool row_rc_fits(const PassDesc& P, bool smooth = false);
+bool row_rc_fits(const PassDesc& P);
 bool col_rc_fits(const PassDesc& P);
-void launch_row_rc(const PassDesc& P, hipStream_t s);
 std::vector<double> row_r2r_table(int kind, int n);
 void launch_row_r2r(const PassDesc& P, hipStream_t s);
 bool col_r2r_fits(const PassDesc& P, bool smooth = false);
@@ -444,15 +443,6 @@ PassDesc SolverImpl::pass_desc(const DirPlan& p, int comp, bool forward, const V
         P.aux = twiddles(P.n);
         return P;
     }
-    // real-to-complex pencils along the contiguous direction: packed half-length FFT in registers
-    if (!std::getenv("FLUPS_GENERIC_PASS") && row_rc_fits(P)) {
-        P.fastk = 3;
-        int pf = 1, q = P.n / 2;
-        split_pq(P.n / 2, pf, q);
-        P.tw = twiddles(q);
-        P.aux = twiddles(P.n);
-        return P;
-    }
     // real-to-complex pencils along a strided direction, neighbours along a unit-stride one:
     // pairs of real pencils as one complex column
     if (!std::getenv("FLUPS_GENERIC_PASS") && col_real_fits(P)) {
@@ -468,7 +458,8 @@ PassDesc SolverImpl::pass_desc(const DirPlan& p, int comp, bool forward, const V
         P.vec = ((uintptr_t)real % (2 * res) == 0) && rs[P.d] % 2 == 0 && rs[P.fb] % 2 == 0 && P.na % 2 == 0;
         return P;
     }
-    // the same shapes at the other lengths with factors 2, 3, 5, 7: run-time mixed radix
+    // contiguous real-to-complex pencils, and the same shapes at the other lengths with factors 2, 3, 5, 7: run-time
+    // mixed radix
     if (!std::getenv("FLUPS_GENERIC_PASS") && smooth_pass(P)) return P;
     P.alias = generic_alias(P) ? 1 : 0;
     const size_t per_pen = generic_lds_bytes(P, 1);
@@ -487,7 +478,7 @@ PassDesc SolverImpl::pass_desc(const DirPlan& p, int comp, bool forward, const V
 // a pass for the kernels of smooth.hip (sm.M > 0): its shape's code, tile and tables (false: none fits)
 bool SolverImpl::smooth_pass(PassDesc& P) {
     PassDesc Q = P;
-    const bool row = row_r2r_fits(P, true) || row_rc_fits(P, true) || row_c2c_fits(P, true);
+    const bool row = row_r2r_fits(P, true) || row_rc_fits(P) || row_c2c_fits(P, true);
     if (row || col_r2r_fits(P, true) || col_rc_fits(P)) {
         const int h = P.op == OP_R2R ? r2r_h(P.kind, P.n) : P.op == OP_C2C ? P.n : P.n / 2;
         if (!smooth_pen_tile(Q, h, !row)) return false;
@@ -537,7 +528,6 @@ void SolverImpl::run_pass(const PassDesc& P) {
     }
     if (P.fastk == 1) launch_row_r2r(P, stream_);
     else if (P.fastk == 2) launch_col_real(P, stream_);
-    else if (P.fastk == 3) launch_row_rc(P, stream_);
     else if (P.fastk == 4) launch_col_r2r(P, stream_);
     else if (P.fastk == 5) launch_col_c2c(P, stream_);
     else if (P.fastk == 6) launch_row_c2c(P, stream_);
