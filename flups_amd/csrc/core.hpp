@@ -144,6 +144,18 @@ struct SmoothZArgs {
     SmoothPlan sm;
 };
 
+// the same for an r2c last direction, pairs of real columns that are neighbours along x (smooth.hip)
+struct SmoothRzArgs {
+    void* d = nullptr;           // field before the transform, in place: (nx, ny, nin) reals, x fastest
+    const void* g = nullptr;     // Green's function on the spectral layout (nx, ny, M/2 + 1) complex
+    const double* tw = nullptr;  // M-point twiddle table
+    int nx = 1, ny = 1, nin = 1, tx = 4, lda = 1;   // tx pairs per block
+    int f32 = 0;                 // data and G stored as float (FP64 arithmetic)
+    long long s_col = 1, comp = 0;
+    double normfact = 1;
+    SmoothPlan sm;
+};
+
 // the same with the curl of three components (smooth_rot.hip)
 struct SmoothRotArgs {
     void* d = nullptr;           // the three components before the transform, in place: complex, x fastest

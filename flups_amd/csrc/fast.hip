@@ -934,6 +934,7 @@ bool row_rz_len_ok(int M);
 bool split_pq(int n, int& pf, int& q);
 int smooth_z_tile(int M, bool f32);                          // smooth.hip
 void launch_smooth_z(const SmoothZArgs& A, hipStream_t s);
+void launch_smooth_rz(const SmoothRzArgs& A, hipStream_t s);
 int smooth_rot_tile(int M, bool f32);                        // smooth_rot.hip
 void launch_smooth_rot(const SmoothRotArgs& A, hipStream_t s);
 
@@ -1011,8 +1012,12 @@ HybridZ* make_hybrid_z(SolverImpl& s) {
         // the Green's function keeps the general path's spectral layout
         const int M = f.n_in[0];
         if (in.nf != 1 || sp.nf != 2 || in.n[0] != sp.n[0] || (nd == 3 && in.n[1] != sp.n[1])) return nullptr;
-        if (!pow2_in(M, 32, 1024) || sp.n[nd - 1] != M / 2 + 1 || in.n[nd - 1] > M || !s.dgreen_) return nullptr;
+        const bool p2 = pow2_in(M, 32, 1024);
+        const int smooth_tx = p2 ? 0 : smooth_z_tile(M, f32);
+        if (!(p2 || smooth_tx) || sp.n[nd - 1] != M / 2 + 1 || in.n[nd - 1] > M || !s.dgreen_) return nullptr;
         auto* h = new HybridZ;
+        h->smooth = !p2;
+        h->gtx = smooth_tx;
         h->f32 = f32;
         h->real = true;
         h->M = M;
@@ -1137,6 +1142,24 @@ void hybrid_z_t(const HybridZ* h, void* data, hipStream_t st) {
         A.comp = (long long)h->nx * h->ny;
         A.normfact = h->normfact;
         launch_row_rz(A, st);
+        return;
+    }
+    if (h->real && h->smooth) {
+        SmoothRzArgs A;
+        A.f32 = std::is_same<S, float>::value;
+        A.d = data;
+        A.g = h->g;
+        A.tw = static_cast<const double*>(h->tw);
+        A.nx = h->nx;
+        A.ny = h->ny;
+        A.nin = h->nz;
+        A.tx = h->gtx;
+        A.lda = h->lda;
+        A.s_col = (long long)h->nx * h->ny;
+        A.comp = (long long)h->nx * h->ny * h->nz;
+        A.normfact = h->normfact;
+        smooth_plan(h->M, A.sm);
+        launch_smooth_rz(A, st);
         return;
     }
     if (h->real) {

@@ -5,6 +5,7 @@
 //   smooth_col   c2c along a strided direction, values straight between HBM and the first / last
 //                stage's registers;
 //   smooth_z     the last direction fused with the multiply: forward c2c, normfact G, inverse c2c;
+//   smooth_rz    the same for an r2c last direction, pairs of real columns;
 //   smooth_pen   every other pass (r2c, c2r, r2r, c2c of a contiguous pencil; r2c, c2r, r2r of a
 //                strided one), pre- and post-maps from tables (smooth_pen.hpp).
 // Before, these lengths ran on the generic kernel (up to five radix 2-7 stages over LDS, sines and
@@ -194,6 +195,116 @@ struct smooth_z {
     }
 };
 
+// An r2c last direction: two neighbouring real columns a, b as one complex column a + i b, whose product
+// spectrum is Z'[k] = (Ga + Gb)/2 Z[k] + (Ga - Gb)/2 conj Z[M-k] (G real and even in kz). The mirrored value
+// lies with another thread: the forward spectrum passes through LDS between the transforms.
+// 129 x 161 x 97 node-centred walls, MI355X: r2c 22, multiply 15 and c2r 23 us before, 27 us now.
+template <bool WIDE, typename ST>
+struct smooth_rz {
+    using Args = SmoothRzArgs;
+    static constexpr int NT = 512, kWaves = WIDE ? 3 : 4;
+    static __device__ __forceinline__ void run(const SmoothRzArgs& A, Blk blk) {
+        extern __shared__ double smem[];
+        C2<double>* lds = reinterpret_cast<C2<double>*>(smem);
+        const SmoothPlan& S = A.sm;
+        const int M = S.M, tx = A.tx;
+        const int c = threadIdx.x & (tx - 1), t = threadIdx.x / tx;
+        const int npair = (A.nx + 1) / 2, ntile = (npair + tx - 1) / tx;
+        const int b = xcd_group(blk.x, blk.nx);
+        const int tile = b % ntile, y = b / ntile;
+        const int pr = tile * tx + c;
+        const bool la = pr < npair;
+        const int xa = 2 * min(pr, npair - 1);   // dead pairs read the last pair and store nothing
+        const bool hb = xa + 1 < A.nx;           // the partner column exists
+        ST* base = reinterpret_cast<ST*>(A.d) + (long long)blk.y * A.comp + (long long)y * A.nx + xa;
+        const ST* g = reinterpret_cast<const ST*>(A.g) + 2 * ((long long)y * A.nx + xa);
+        const long long gs = 2LL * A.nx * A.ny;   // reals between kz rows of G
+        const C2<double>* tw = reinterpret_cast<const C2<double>*>(A.tw);
+        auto slot = [&](int e) { return e * tx + c; };
+        auto ext = [&](C2<double>* v, int mp, auto r) {
+            constexpr int R = decltype(r)::value;
+            const ST* p = base + t * A.s_col;
+            const long long step = mp * A.s_col;
+#pragma unroll
+            for (int q = 0; q < R; ++q) {
+                v[q] = {0.0, 0.0};
+                if (t + q * mp < A.nin) v[q] = {(double)p[q * step], hb ? (double)p[q * step + 1] : 0.0};
+            }
+        };
+        auto out = [&](C2<double>* v, int mp, auto r) {
+            constexpr int R = decltype(r)::value;
+            if (!la) return;
+            ST* p = base + t * A.s_col;
+            const long long step = mp * A.s_col;
+#pragma unroll
+            for (int u = 0; u < R; ++u)
+                if (t + u * mp < A.nin) {
+                    p[u * step] = (ST)v[u].y;
+                    if (hb) p[u * step + 1] = (ST)v[u].x;
+                }
+        };
+        auto none = [](C2<double>*, int, auto) {};
+        const int last = S.nst - 1;
+#define FLUPS_CALL(R) smooth_stage<R>(t, S.mp[0], 1, S.inv[0], S.stride[0], true, false, lds, slot, tw, ext, none)
+        FLUPS_SMOOTH_RADIX(S.rad[0], FLUPS_CALL)
+#undef FLUPS_CALL
+        for (int s = 1; s < last; ++s) {
+#define FLUPS_CALL(R) smooth_stage<R>(t, S.mp[s], S.span[s], S.inv[s], S.stride[s], false, false, lds, slot, tw, none, none)
+            FLUPS_SMOOTH_RADIX(S.rad[s], FLUPS_CALL)
+#undef FLUPS_CALL
+        }
+        auto middle = [&](auto r) {
+            constexpr int R = decltype(r)::value;
+            const int mp = S.mp[last];
+            const bool on = t < mp;
+            C2<double> v[R];
+            double ga[R], gb[R];
+            if (on) {
+#pragma unroll
+                for (int u = 0; u < R; ++u) {
+                    const int k = t + u * mp, kz = min(k, M - k);
+                    ga[u] = (double)g[kz * gs];
+                    gb[u] = hb ? (double)g[kz * gs + 2] : ga[u];
+                }
+#pragma unroll
+                for (int q = 0; q < R; ++q) v[q] = lds[slot(t + q * mp)];
+                twiddle_r<R>(v, tw, t);
+                dft_r<R>(v);
+#pragma unroll
+                for (int u = 0; u < R; ++u) lds[slot(t + u * mp)] = v[u];   // X[t + u mp], the thread's own slots
+            }
+            __syncthreads();
+            if (on) {
+#pragma unroll
+                for (int u = 0; u < R; ++u) {
+                    const int k = t + u * mp;
+                    const C2<double> zc = cconj(lds[slot(k == 0 ? 0 : M - k)]);
+                    const double p = 0.5 * (ga[u] + gb[u]) * A.normfact, q = 0.5 * (ga[u] - gb[u]) * A.normfact;
+                    v[u] = {p * v[u].y + q * zc.y, p * v[u].x + q * zc.x};   // swapped: inverse
+                }
+                dft_r<R>(v);
+            }
+            __syncthreads();   // the mirrored values are read
+            if (on) {
+#pragma unroll
+                for (int u = 0; u < R; ++u) lds[slot(t * R + u)] = v[u];
+            }
+            __syncthreads();
+        };
+#define FLUPS_CALL(R) middle(std::integral_constant<int, R>{})
+        FLUPS_SMOOTH_RADIX(S.rad[last], FLUPS_CALL)
+#undef FLUPS_CALL
+        for (int s = last - 1; s > 0; --s) {
+#define FLUPS_CALL(R) smooth_stage<R>(t, S.mp[s], S.rspan[s], S.rinv[s], S.rstride[s], false, false, lds, slot, tw, none, none)
+            FLUPS_SMOOTH_RADIX(S.rad[s], FLUPS_CALL)
+#undef FLUPS_CALL
+        }
+#define FLUPS_CALL(R) smooth_stage<R>(t, S.mp[0], S.rspan[0], S.rinv[0], S.rstride[0], false, true, lds, slot, tw, none, out)
+        FLUPS_SMOOTH_RADIX(S.rad[0], FLUPS_CALL)
+#undef FLUPS_CALL
+    }
+};
+
 constexpr size_t kSmoothLds = 65536;   // bytes of one block
 constexpr int kSmoothThreads = 512;
 
@@ -324,6 +435,14 @@ void launch_smooth_z(const SmoothZArgs& A, hipStream_t s) {
     const size_t lds = (size_t)A.tx * A.sm.M * 2 * sizeof(double);
     if (A.f32) A.sm.wide ? launch_k<smooth_z<true, float>>(grid, block, lds, s, A) : launch_k<smooth_z<false, float>>(grid, block, lds, s, A);
     else A.sm.wide ? launch_k<smooth_z<true, double>>(grid, block, lds, s, A) : launch_k<smooth_z<false, double>>(grid, block, lds, s, A);
+    HIP_CHECK(hipGetLastError());
+}
+
+void launch_smooth_rz(const SmoothRzArgs& A, hipStream_t s) {
+    const dim3 grid(((A.nx + 1) / 2 + A.tx - 1) / A.tx * A.ny, A.lda), block(A.tx * A.sm.T);
+    const size_t lds = (size_t)A.tx * A.sm.M * 2 * sizeof(double);
+    if (A.f32) A.sm.wide ? launch_k<smooth_rz<true, float>>(grid, block, lds, s, A) : launch_k<smooth_rz<false, float>>(grid, block, lds, s, A);
+    else A.sm.wide ? launch_k<smooth_rz<true, double>>(grid, block, lds, s, A) : launch_k<smooth_rz<false, double>>(grid, block, lds, s, A);
     HIP_CHECK(hipGetLastError());
 }
 
