@@ -31,13 +31,15 @@ void launch_smooth_tile(const PassDesc& P, dim3 grid, dim3 block, size_t lds, hi
 
 namespace {
 
-// WIDE: radices up to 16 (two stages for most lengths up to 256) in 128 registers; otherwise up to 10
-// in 80 registers, six waves per SIMD: with three stages the barriers between them want the waves
-// (200 x 144 x 100 open: fused z 131 us with every radix in one kernel, 84 us so; y 47 -> 32 us)
+// WIDE: radices up to 16 (two stages for most lengths up to 256) in 168 registers, three waves per SIMD: at
+// 128 they spilled 20 to 40 (120^3 open 140 -> 126 us, 240^3 periodic 349 -> 316), and a block of
+// 64 threads and 12 KB of LDS reaches no fourth wave. Otherwise up to 10 in 80 registers, six waves: with three
+// stages the barriers between them want the waves (200 x 144 x 100 open: fused z 131 us with every
+// radix in one kernel, 84 us so; five waves 193 -> 199, seven 196, eight 225 us the solve)
 template <bool WIDE, typename TI, typename TO>
 struct smooth_col {
     using Args = PassDesc;
-    static constexpr int NT = 512, kWaves = WIDE ? 4 : 6;
+    static constexpr int NT = 512, kWaves = WIDE ? 3 : 6;
     static __device__ __forceinline__ void run(const PassDesc& P, Blk blk) {
         extern __shared__ double smem[];
         C2<double>* lds = reinterpret_cast<C2<double>*>(smem);
@@ -103,7 +105,7 @@ struct smooth_col {
 template <bool WIDE, typename ST>
 struct smooth_z {
     using Args = SmoothZArgs;
-    static constexpr int NT = 512, kWaves = WIDE ? 4 : 6;
+    static constexpr int NT = 512, kWaves = WIDE ? 3 : 6;
     static __device__ __forceinline__ void run(const SmoothZArgs& A, Blk blk) {
         extern __shared__ double smem[];
         C2<double>* lds = reinterpret_cast<C2<double>*>(smem);
