@@ -198,7 +198,7 @@ struct smooth_z {
 };
 
 // An r2c last direction: two neighbouring real columns a, b as one complex column a + i b, whose product
-// spectrum is Z'[k] = (Ga + Gb)/2 Z[k] + (Ga - Gb)/2 conj Z[M-k] (G real and even in kz). The mirrored value
+// spectrum is Z'[k] = Ga/2 (Z[k] + conj Z[M-k]) + Gb/2 (Z[k] - conj Z[M-k]) (G real and even in kz). The mirrored value
 // lies with another thread: the forward spectrum passes through LDS between the transforms.
 // 129 x 161 x 97 node-centred walls, MI355X: r2c 22, multiply 15 and c2r 23 us before, 27 us now.
 template <bool WIDE, typename ST>
@@ -281,8 +281,9 @@ struct smooth_rz {
                 for (int u = 0; u < R; ++u) {
                     const int k = t + u * mp;
                     const C2<double> zc = cconj(lds[slot(k == 0 ? 0 : M - k)]);
-                    const double p = 0.5 * (ga[u] + gb[u]) * A.normfact, q = 0.5 * (ga[u] - gb[u]) * A.normfact;
-                    v[u] = {p * v[u].y + q * zc.y, p * v[u].x + q * zc.x};   // swapped: inverse
+                    const C2<double> s = cadd(v[u], zc), d = csub(v[u], zc);
+                    const double p = 0.5 * A.normfact * ga[u], q = 0.5 * A.normfact * gb[u];
+                    v[u] = {p * s.y + q * d.y, p * s.x + q * d.x};   // swapped: inverse
                 }
                 dft_r<R>(v);
             }
