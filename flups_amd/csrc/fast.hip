@@ -940,7 +940,7 @@ int smooth_z_tile(int M, bool f32);                          // smooth.hip
 void launch_smooth_z(const SmoothZArgs& A, hipStream_t s);
 void launch_smooth_rz(const SmoothRzArgs& A, hipStream_t s);
 int smooth_rot_tile(int M, bool f32);                        // smooth_rot.hip
-void launch_smooth_rot(const SmoothRotArgs& A, hipStream_t s);
+void launch_smooth_rot(SmoothRotArgs A, hipStream_t s);
 
 struct HybridZ {
     int M = 0, nx = 0, ny = 0, nz = 0, lda = 1, gtx = 8;
@@ -1262,7 +1262,7 @@ void hybrid_z(const HybridZ* h, void* data, int type, hipStream_t st) {
         A.s_col = (long long)h->nx * h->ny;
         A.s_other = h->nx;
         A.comp = (long long)h->nx * h->ny * h->nz;
-        smooth_plan(h->M, A.sm);
+        A.sm.M = h->M;   // the launch chooses the stages
         launch_smooth_rot(A, st);
         return;
     }

@@ -336,7 +336,7 @@ int col_tile(int M, int T, bool f32) {
 // fewest stages, then radices up to 10 (the kernels with fewer registers), then fewest threads (the
 // largest smallest radix); radices ascending, so that every thread takes part in the first stage and in
 // the last one of a fused inverse, the ones that meet HBM
-static bool search_plan(int M, SmoothPlan& p) {
+static bool search_plan(int M, int maxrad, SmoothPlan& p) {
     static const int rads[13] = {2, 3, 4, 5, 6, 7, 8, 9, 10, 12, 14, 15, 16};
     std::vector<int> cur, best;
     auto search = [&](auto&& self, int m, int lo) -> void {
@@ -350,7 +350,7 @@ static bool search_plan(int M, SmoothPlan& p) {
         }
         if ((int)cur.size() == kSmoothStages) return;
         for (int i = lo; i < 13; ++i)
-            if (m % rads[i] == 0) {
+            if (m % rads[i] == 0 && rads[i] <= maxrad) {
                 cur.push_back(rads[i]);
                 self(self, m / rads[i], i);
                 cur.pop_back();
@@ -381,21 +381,24 @@ static bool search_plan(int M, SmoothPlan& p) {
     }
     return p.T <= kSmoothThreads;
 }
-// every pass of every solve asks: the answers (a function of M alone, at most 2031 of them) are kept
-bool smooth_plan(int M, SmoothPlan& p) {
+// every pass of every solve asks: the answers (a function of M and of the largest radix alone, a few thousand
+// at most) are kept
+bool smooth_plan_upto(int M, int maxrad, SmoothPlan& p) {
     if (M < 16 || M > 2048) return false;
     static std::mutex mu;
-    static std::map<int, SmoothPlan> known;   // M = 0: no plan
+    static std::map<std::pair<int, int>, SmoothPlan> known;   // M = 0: no plan
     std::lock_guard<std::mutex> lk(mu);
-    auto it = known.find(M);
+    const auto key = std::make_pair(M, maxrad);
+    auto it = known.find(key);
     if (it == known.end()) {
         SmoothPlan q;
-        if (!search_plan(M, q)) q = SmoothPlan();
-        it = known.emplace(M, q).first;
+        if (!search_plan(M, maxrad, q)) q = SmoothPlan();
+        it = known.emplace(key, q).first;
     }
     p = it->second;
     return p.M == M;
 }
+bool smooth_plan(int M, SmoothPlan& p) { return smooth_plan_upto(M, 16, p); }
 
 bool smooth_col_tile(PassDesc& P, int n) {
     if (!smooth_plan(n, P.sm)) return false;

@@ -8,7 +8,7 @@
 // component's LDS reads and its writes lies one barrier, which also orders the component before it, so a
 // stage costs three barriers for three transforms. The last forward stage, the curl and the
 // first inverse stage (the same radix) touch a thread's own LDS slots only. 160^3 layer, FP32
-// storage, MI355X: 3 x 30 + 70 + 3 x 30 us -> 145 us, the solve 556 -> 450 us.
+// storage, MI355X: 3 x 30 + 70 + 3 x 30 us -> 149 us, the solve 556 -> 450 us.
 #include <hip/hip_runtime.h>
 
 #include "core.hpp"
@@ -18,14 +18,17 @@
 
 namespace flups {
 
+bool smooth_plan_upto(int M, int maxrad, SmoothPlan& p);   // smooth.hip
+
 namespace {
 
-// WIDE: radices up to 16, else up to 10. Registers for two or three waves per SIMD: the LDS of three
-// components holds a CU to about 52 / (smallest radix) waves anyway
-template <bool WIDE, typename ST>
+// Registers for three waves per SIMD: the LDS of three components holds a CU to about 52 / (smallest radix)
+// waves anyway
+template <typename ST>
 struct smooth_rot {
     using Args = SmoothRotArgs;
-    static constexpr int NT = 512, kWaves = WIDE ? 2 : 3;
+    static constexpr int NT = 512, kWaves = 3;
+    static constexpr bool WIDE = false;   // radices up to 10 (rot_plan)
     static __device__ __forceinline__ void run(const SmoothRotArgs& A, Blk blk) {
         extern __shared__ double smem[];
         const SmoothPlan& S = A.sm;
@@ -163,22 +166,28 @@ struct smooth_rot {
 // 161 us (8 -> 4 columns), 160^3 open 1103 -> 1093 (4 -> 2), 160^3 layer 365 -> 361; 32 KB: batch 1548 -> 1635
 constexpr size_t kRotLds = 54272;
 
+// Radices up to 10 where the tile's LDS limits the waves: 112^3 open 389 -> 367 us, layer 157 -> 143, 96^3 layer 107 ->
+// 95, 32 mixed problems 1555 -> 1525 against up to 16 (two stages, but three blocks of 64 threads a
+// CU); up to 8 the same within 1 %, up to 6 slower (80^3 open 153 -> 254). Every length that fits has such a plan.
+bool rot_plan(int M, SmoothPlan& p) { return smooth_plan_upto(M, 10, p); }
+
 }  // namespace
 
 // columns per block (0: no kernel for this length)
 int smooth_rot_tile(int M, bool f32) {
     SmoothPlan p;
-    if (!smooth_plan(M, p)) return 0;
+    if (!rot_plan(M, p)) return 0;
     int tx = f32 ? 8 : 4;
     while (tx * p.T < 64) tx *= 2;
     while (tx > 1 && (tx * p.T > 512 || (size_t)3 * M * tx * sizeof(C2<double>) > kRotLds)) tx /= 2;
     return tx * p.T <= 512 && (size_t)3 * M * tx * sizeof(C2<double>) <= kRotLds ? tx : 0;
 }
-void launch_smooth_rot(const SmoothRotArgs& A, hipStream_t s) {
+void launch_smooth_rot(SmoothRotArgs A, hipStream_t s) {
+    FLUPS_REQUIRE(rot_plan(A.sm.M, A.sm), "no stages for columns of %d points", A.sm.M);
     const dim3 grid((A.nx + A.tx - 1) / A.tx * A.nother), block(A.tx * A.sm.T);
     const size_t lds = (size_t)3 * A.tx * A.sm.M * sizeof(C2<double>);
-    if (A.f32) A.sm.wide ? launch_k<smooth_rot<true, float>>(grid, block, lds, s, A) : launch_k<smooth_rot<false, float>>(grid, block, lds, s, A);
-    else A.sm.wide ? launch_k<smooth_rot<true, double>>(grid, block, lds, s, A) : launch_k<smooth_rot<false, double>>(grid, block, lds, s, A);
+    if (A.f32) launch_k<smooth_rot<float>>(grid, block, lds, s, A);
+    else launch_k<smooth_rot<double>>(grid, block, lds, s, A);
     HIP_CHECK(hipGetLastError());
 }
 
