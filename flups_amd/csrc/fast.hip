@@ -842,11 +842,11 @@ void run_fast(FastPlan* f, void* s0, void* s1, const double* rhs, double* field,
         z.comp_src = c1;
         z.comp_dst = c1;
         z.xcd = (f->zsched >> 4) & 1;
-        // the two rows of a mirror pair in one block (one read of G's slice), or in neighbouring blocks where the
-        // pairs are less than three rounds of the chip's waves (16 on each of 256 CUs; 64^3 open 41.0 -> 40.0, 128^3
-        // 100 -> 98.5, 128 x 128 x 256 195 -> 197 us)
-        const double waves = (double)((z.nx + f->gtx - 1) / f->gtx) * z.gy * f->lda * f->gtx * M2 / 512;
-        z.nopair = (f->zsched & 32) || ((f->zsched & 3) == 0 && waves < 3 * 16 * 256) ? 2 : 0;
+        // the two rows of a mirror pair in one block (one read of G's slice); bit 5: in neighbouring blocks. What
+        // the schedule says and nothing else: the neighbours are faster where the field is small (open 32^3 26.4 -> 25.1,
+        // 64^3 40.7 -> 40.0, 128^3 100.1 -> 98.4 us; three components of 128^3 281.6 -> 285.7) and slower
+        // from 128 x 128 x 256 on (195 -> 197)
+        z.nopair = (f->zsched & 32) ? 2 : 0;
         z.x0 = x0;
         z.gntx = (f->nx + f->gtx - 1) / f->gtx;
         if (type == 1) {

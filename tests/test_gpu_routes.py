@@ -1,0 +1,76 @@
+"""Which kernels a solve launches: the z pass of the fused pipeline under each schedule (row pairs in one block or
+not), and the fused rotational last direction of the general path."""
+import ctypes
+
+import numpy as np
+import pytest
+
+try:
+    import torch  # noqa: F401
+except Exception:   # pragma: no cover
+    torch = None
+
+import flups_amd as fl
+
+pytestmark = pytest.mark.gpu
+
+U = 4
+
+
+class KernelNode(ctypes.Structure):   # hipKernelNodeParams
+    _fields_ = [("block", ctypes.c_uint * 3), ("extra", ctypes.c_void_p), ("func", ctypes.c_void_p), ("grid", ctypes.c_uint * 3),
+                ("params", ctypes.c_void_p), ("shared", ctypes.c_uint)]
+
+
+def grids(solver, nglob):
+    """x extents of the grids of one solve's launches, in order: a captured flups_solve_noalloc"""
+    hip = fl.lib()   # the HIP runtime that the library is linked with
+    stream = fl.Stream()
+    solver.set_stream(stream)
+    h = ctypes.c_void_p(stream.handle)
+    din, dout = fl.DeviceArray((1,) + nglob[::-1]), fl.DeviceArray((1,) + nglob[::-1])
+    graph, n = ctypes.c_void_p(), ctypes.c_size_t(0)
+    assert hip.hipStreamBeginCapture(h, 2) == 0
+    hip.flups_clear_last_error()
+    hip.flups_solve_noalloc(solver._solver, dout.ptr, din.ptr, 0)
+    err = fl.last_error()
+    assert hip.hipStreamEndCapture(h, ctypes.byref(graph)) == 0
+    assert err == "", err
+    assert hip.hipGraphGetNodes(graph, None, ctypes.byref(n)) == 0
+    nodes = (ctypes.c_void_p * n.value)()
+    assert hip.hipGraphGetNodes(graph, nodes, ctypes.byref(n)) == 0
+    out = []
+    for node in nodes:
+        k = KernelNode()
+        assert hip.hipGraphKernelNodeGetParams(ctypes.c_void_p(node), ctypes.byref(k)) == 0
+        out.append(int(k.grid[0]))
+    assert hip.hipGraphDestroy(graph) == 0
+    solver.set_stream(None)
+    return out
+
+
+@pytest.mark.parametrize("nglob", [(32, 32, 32), (64, 64, 64), (128, 64, 32)])
+def test_schedule_is_what_runs(monkeypatch, nglob):
+    """bit 5 of the z schedule and nothing else decides between row pairs in one block and rows in neighbouring blocks, and
+    the schedule that a solver reports launches what the solver launches"""
+    def run(env):
+        for k in ("FLUPS_ZSCHED", "FLUPS_YSCHED", "FLUPS_ORDER", "FLUPS_SLAB_MB"):
+            monkeypatch.delenv(k, raising=False)
+        for k, v in env.items():
+            monkeypatch.setenv(k, str(v))
+        s = fl.Solver(fl.Topology(0, 1, list(nglob), [1, 1, 1], False), [[U, U]] * 3, [1.0 / 64] * 3, [n / 64 for n in nglob])
+        s.set_green_type(2)
+        s.setup()
+        assert s.path == 1
+        return grids(s, nglob), s.schedule
+
+    default, sched = run({})
+    assert len(default) == 5
+    assert run({"FLUPS_ZSCHED": sched[0]})[0] == default
+    for z in (0, 4, 8, 16, 20):
+        pair, single = run({"FLUPS_ZSCHED": z})[0], run({"FLUPS_ZSCHED": z | 32})[0]
+        assert single[2] == 2 * pair[2], (z, pair, single)
+    # x slabs (whole tiles): as many blocks in all as the whole field takes
+    slabs = run({"FLUPS_SLAB_MB": 0.25, "FLUPS_ZSCHED": 20})[0]
+    assert len(slabs) > 5
+    assert sum(slabs[2:-1:3]) == default[2], (slabs, default)
