@@ -131,6 +131,15 @@ struct PassDesc {
     __host__ __device__ T* to(int c) const { return reinterpret_cast<T*>(dst) + c * dst_c; }
 };
 
+// how the general path fuses a c2c last direction with the multiply (gtx = 0: it does not)
+struct HybridC2C {
+    int gtx = 0, gy = 0;   // tile width and rows of the compressed Green's function
+    bool p2 = false;       // power of two: z_fused, else smooth_z
+    bool pair = false;     // rows y and M1 - y share their G
+    int rtx = 0;           // columns per block of the rotational pass (0: not fused)
+    size_t green = 0;      // reals of the compressed Green's function
+};
+
 // the last direction of the general path, c2c of a smooth length, with the multiply (smooth.hip)
 struct SmoothZArgs {
     void* d = nullptr;           // field before the transform, in place: complex, x fastest, rows s_col apart

@@ -960,20 +960,58 @@ struct HybridZ {
     double bytes = 0;        // algorithmic bytes of one launch
 };
 
-HybridZ* make_hybrid_z(SolverImpl& s) {
-    const int nd = s.ndim_;
-    if (nd != 3 && nd != 2) return nullptr;
-    const bool f32 = s.gf32_;           // the general path's FP32 solves: float data and Green's function
-    const double es = f32 ? 4.0 : 8.0;   // bytes of one stored real
-    if (getenv("FLUPS_FORCE_GENERIC")) return nullptr;
-    const int ip = nd - 1;
-    const DirPlan &f = s.fwd_[ip], &b = s.bwd_[ip];
-    if (!(f.type == UNBUNB || (f.type == PERPER && !s.node_))) return nullptr;
-    if (f.dim != nd - 1 && !(f.dim == 0 && f.r2c)) return nullptr;
+// the last direction is an unbounded or cell-centred periodic one without offsets or post-corrections
+static bool plain_last(const DirPlan& f, const DirPlan& b, int nd, bool node) {
+    if (nd != 3 && nd != 2) return false;
+    if (getenv("FLUPS_FORCE_GENERIC")) return false;
+    if (!(f.type == UNBUNB || (f.type == PERPER && !node))) return false;
+    if (f.dim != nd - 1 && !(f.dim == 0 && f.r2c)) return false;
     for (const DirPlan* p : {&f, &b})
         for (int c = 0; c < p->lda; ++c)
             if (p->post[c] != 0 || p->start_in[c] != 0 || p->start_out[c] != 0 || p->fieldstart != 0 || p->koffset != 0.0)
-                return nullptr;
+                return false;
+    return true;
+}
+
+HybridC2C plan_hybrid_c2c(const SolverImpl& s, bool f32) {
+    HybridC2C r;
+    const int nd = s.ndim_;
+    const DirPlan& f = s.fwd_[nd - 1];
+    if (!plain_last(f, s.bwd_[nd - 1], nd, s.node_) || f.r2c) return r;
+    const Shape &in = s.stage_[nd - 2], &sp = s.stage_[nd - 1];
+    const int M = f.n_in[0], ny = nd == 3 ? in.n[1] : 1;
+    if (in.nf != 2 || sp.nf != 2 || in.n[0] != sp.n[0] || (nd == 3 && in.n[1] != sp.n[1]) || sp.n[nd - 1] != M) return r;
+    if ((double)(M / 8) * in.n[0] * ny * 16.0 >= 4294967296.0) return r;
+    // powers of two in registers (half-width x tiles in 3-D; two columns per block in 2-D: few columns, cache-resident
+    // field); 3, 5, 7 times one on smooth_z as well (open 160^3 389 -> 338, 224^3 1032 -> 931, 48^3 70 -> 57 us against
+    // register columns and thread teams)
+    r.p2 = pow2_in(M, 32, nd == 2 ? 2048 : 1024);
+    r.gtx = !r.p2 ? smooth_z_tile(M, f32) : nd == 2 ? 2 : 4;
+    if (!r.gtx) return r;
+    // y rows pair as (y, M1 - y) when y is a full unbounded / periodic c2c direction (G even in ky)
+    const DirPlan& fy = s.fwd_[1];
+    r.pair = nd == 3 && fy.dim == 1 && !fy.r2c && (fy.type == UNBUNB || (fy.type == PERPER && !s.node_)) && fy.koffset == 0.0 &&
+             fy.n_in[0] == ny;
+    r.gy = r.pair ? ny / 2 + 1 : ny;
+    r.green = (size_t)r.gy * ((in.n[0] + r.gtx - 1) / r.gtx) * (M / 2 + 1) * r.gtx;
+    // the rotational pass: every direction unbounded or periodic, so that each derivative is i K with
+    // the same real K for the three components
+    bool rot = nd == 3 && s.lda_ == 3 && s.odiff_ != NOD;
+    for (int i = 0; i < nd && rot; ++i) {
+        const DirPlan& p = s.fwd_[i];
+        rot = (p.type == UNBUNB || p.type == PERPER) && p.koffset == 0.0;
+        for (int c = 0; c < 3; ++c) rot = rot && s.bwdd_[i].imult[c] == p.imult[c];
+    }
+    if (rot) r.rtx = smooth_rot_tile(M, f32);
+    return r;
+}
+
+HybridZ* make_hybrid_z(SolverImpl& s) {
+    const int nd = s.ndim_;
+    const bool f32 = s.gf32_;           // the general path's FP32 solves: float data and Green's function
+    const double es = f32 ? 4.0 : 8.0;   // bytes of one stored real
+    if (!plain_last(s.fwd_[nd - 1], s.bwd_[nd - 1], nd, s.node_)) return nullptr;
+    const DirPlan& f = s.fwd_[nd - 1];
     const Shape& in = s.stage_[nd - 2];   // field before the last transform
     const Shape& sp = s.stage_[nd - 1];   // spectral field (and Green's function)
     if (f.r2c && f.dim == 0) {
@@ -1044,34 +1082,24 @@ HybridZ* make_hybrid_z(SolverImpl& s) {
         h->bytes = h->lda * 2.0 * (double)h->nx * h->ny * h->nz * es + (double)h->nx * h->ny * (M / 2 + 1) * 2 * es;
         return h;
     }
-    if (in.nf != 2 || sp.nf != 2 || in.n[0] != sp.n[0] || (nd == 3 && in.n[1] != sp.n[1])) return nullptr;
+    const HybridC2C plan = plan_hybrid_c2c(s, f32);
+    if (!plan.gtx) return nullptr;
     const int M = f.n_in[0];
-    // powers of two in registers; 3, 5, 7 times one on smooth_z as well (open 160^3 389 -> 338, 224^3 1032 -> 931,
-    // 48^3 70 -> 57 us against register columns and thread teams)
-    const bool p2 = pow2_in(M, 32, nd == 2 ? 2048 : 1024);
-    const int smooth_tx = p2 ? 0 : smooth_z_tile(M, f32);
-    if (!(p2 || smooth_tx) || sp.n[nd - 1] != M) return nullptr;
-    const int ny = nd == 3 ? in.n[1] : 1;
-    if ((double)(M / 8) * in.n[0] * ny * 16.0 >= 4294967296.0) return nullptr;
     auto* h = new HybridZ;
     h->f32 = f32;
     h->M = M;
     h->nx = in.n[0];
-    h->ny = ny;
+    h->ny = nd == 3 ? in.n[1] : 1;
     h->nz = in.n[nd - 1];
     h->lda = s.lda_;
-    // y rows pair as (y, M1 - y) when y is a full unbounded / periodic c2c direction (G even in ky)
-    const DirPlan& fy = s.fwd_[1];
-    h->pair = nd == 3 && fy.dim == 1 && !fy.r2c && (fy.type == UNBUNB || (fy.type == PERPER && !s.node_)) &&
-              fy.koffset == 0.0 && fy.n_in[0] == h->ny;
-    // half-width x tiles in 3-D; two columns per block in 2-D (few columns, cache-resident field)
-    h->gtx = nd == 2 ? 2 : 4;
+    h->pair = plan.pair;
+    h->gtx = plan.gtx;
+    h->rtx = plan.rtx;
     h->twod = nd == 2;
-    h->smooth = !p2;
-    if (h->smooth) h->gtx = smooth_tx;
+    h->smooth = !plan.p2;
     const int ntx = (h->nx + h->gtx - 1) / h->gtx;
-    const int gy = h->pair ? h->ny / 2 + 1 : h->ny, gz = M / 2 + 1;
-    const size_t gn = (size_t)gy * ntx * gz * h->gtx;
+    const int gy = plan.gy, gz = M / 2 + 1;
+    const size_t gn = plan.green;
     try {
         HIP_CHECK(hipMalloc(&h->green, gn * (size_t)es));
         h->dev_bytes += gn * (size_t)es;
@@ -1082,19 +1110,14 @@ HybridZ* make_hybrid_z(SolverImpl& s) {
         HIP_CHECK(hipMalloc(&h->tw, t.size() * sizeof(double)));
         HIP_CHECK(hipMemcpy(h->tw, t.data(), t.size() * sizeof(double), hipMemcpyHostToDevice));
         h->dev_bytes += t.size() * sizeof(double);
-        // the rotational pass: every direction unbounded or periodic, so that each derivative is i K with
-        // the same real K for the three components
-        bool rot = nd == 3 && s.lda_ == 3 && s.odiff_ != NOD;
-        RotK rk{};
-        for (int i = 0; i < nd && rot; ++i) {
-            const DirPlan& p = s.fwd_[i];
-            rot = (p.type == UNBUNB || p.type == PERPER) && p.koffset == 0.0;
-            for (int c = 0; c < 3; ++c) rot = rot && s.bwdd_[i].imult[c] == p.imult[c];
-            rk.kfact[p.dim] = p.kfact;
-            rk.symstart[p.dim] = p.symstart;
-            rk.h[p.dim] = s.h_[p.dim];
-        }
-        if (rot && (h->rtx = smooth_rot_tile(M, f32)) > 0) {
+        if (h->rtx > 0) {   // derivative symbols of the rotational pass
+            RotK rk{};
+            for (int i = 0; i < nd; ++i) {
+                const DirPlan& p = s.fwd_[i];
+                rk.kfact[p.dim] = p.kfact;
+                rk.symstart[p.dim] = p.symstart;
+                rk.h[p.dim] = s.h_[p.dim];
+            }
             rk.order = s.odiff_;
             std::vector<double> t3;
             for (int d = 0; d < 3; ++d)

@@ -59,6 +59,7 @@ void fast_solve_on(FastPlan* f, void* s0, void* s1, double* field, const double*
 void scratch_init();                           // scratch.hip
 double* scratch_device_ptr(size_t* bytes);
 HybridZ* make_hybrid_z(SolverImpl& s);
+HybridC2C plan_hybrid_c2c(const SolverImpl& s, bool f32);
 void destroy_hybrid_z(HybridZ* h);
 size_t hybrid_device_bytes(const HybridZ* h);
 double hybrid_bytes(const HybridZ* h);
@@ -791,10 +792,7 @@ void SolverImpl::setup() {
         dgreen_ = nullptr;
     }
     if (!fast_) {
-        for (int ip = 0; ip < ndim_; ++ip) {
-            const size_t n = std::max(hat_[ip].count(), stage_[ip].count());
-            HIP_CHECK(hipMalloc(&dstage_[ip], n * ses_));
-        }
+        alloc_stages();
         warm_tables();
         warmed_ = true;
     }
@@ -802,6 +800,20 @@ void SolverImpl::setup() {
     HIP_CHECK(hipStreamSynchronize(stream_));
     setup_done_ = true;
     if (prof_) prof_->add("setup", std::chrono::duration<double>(std::chrono::steady_clock::now() - t_setup).count(), 0.0);
+}
+
+// every solve type that this solver takes runs the fused last direction
+bool SolverImpl::fused_only() const {
+    return hybrid_ && hybrid_runs(hybrid_, 0) && (lda_ != 3 || odiff_ == NOD || hybrid_runs(hybrid_, 1));
+}
+
+// the general path's stage arrays; the last one holds the spectral field, which a fused last direction never stores (the
+// advanced interface keeps it in the caller's buffer)
+void SolverImpl::alloc_stages() {
+    for (int ip = 0; ip < ndim_ - (fused_only() ? 1 : 0); ++ip) {
+        const size_t n = std::max(hat_[ip].count(), stage_[ip].count());
+        HIP_CHECK(hipMalloc(&dstage_[ip], n * ses_));
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -915,12 +927,7 @@ void SolverImpl::prepare_advanced() {
     FLUPS_REQUIRE(setup_done_, "flups_setup must be called first");
     FLUPS_REQUIRE(!gf32_, "the advanced interface works on FP64 buffers: this solver was set up for FP32 "
                           "(flups_set_precision(s, 1)) and keeps FP32 stage arrays");
-    if (!dstage_[0]) {
-        for (int ip = 0; ip < ndim_; ++ip) {
-            const size_t m = std::max(hat_[ip].count(), stage_[ip].count());
-            HIP_CHECK(hipMalloc(&dstage_[ip], m * ses_));
-        }
-    }
+    if (!dstage_[0]) alloc_stages();
     if (!dgreen_) compute_green();   // the fused pipeline released the full Green's function
 }
 
@@ -1001,12 +1008,7 @@ void SolverImpl::check_type(int type) const {
 void SolverImpl::prepare(int type) {
     check_type(type);
     if (fast_ && (type == 0 || lda_ == 3)) return;
-    if (!dstage_[0]) {
-        for (int ip = 0; ip < ndim_; ++ip) {
-            const size_t m = std::max(hat_[ip].count(), stage_[ip].count());
-            HIP_CHECK(hipMalloc(&dstage_[ip], m * ses_));
-        }
-    }
+    if (!dstage_[0]) alloc_stages();
     if (!warmed_) {
         warm_tables();
         warmed_ = true;
@@ -1140,7 +1142,11 @@ size_t SolverImpl::predicted_device_bytes(int type) const {
         stages += std::max(hat_[ip].count(), stage_[ip].count());
     }
     const size_t setup_peak = 2 * cap * sizeof(double);
-    const size_t steady = (gpost_[ndim_ - 1].count() + stages) * sizeof(double);
+    // a fused last direction keeps its compressed Green's function in the place of the last stage array, or
+    // beside it where the rotational solves are not fused
+    const HybridC2C h = plan_hybrid_c2c(*this, fp32_);
+    const bool both = h.gtx > 0 && lda_ == 3 && odiff_ != NOD && h.rtx == 0;
+    const size_t steady = (gpost_[ndim_ - 1].count() + stages + (both ? h.green : 0)) * sizeof(double);
     (void)type;
     return std::max(setup_peak, steady) + (size_t)(4u << 20);   // + twiddle tables, LGF tables, slack
 }

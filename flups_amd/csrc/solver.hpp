@@ -122,6 +122,8 @@ class SolverImpl {
     void multiply(void* spec, int type);
     void backward_passes(const void* spec, const View& uout, bool diff);
     void prepare_advanced();
+    bool fused_only() const;
+    void alloc_stages();
     void warm_tables();
     void launch_graph(double* field, const double* rhs, int type);
     void check_type(int type) const;
@@ -170,6 +172,7 @@ class SolverImpl {
     friend FastPlan* make_fast_plan(SolverImpl&);
     friend void build_fast_plan(SolverImpl&, FastPlan*, size_t, int);
     friend HybridZ* make_hybrid_z(SolverImpl&);
+    friend HybridC2C plan_hybrid_c2c(const SolverImpl&, bool);
 };
 
 std::string kernel_dir();
