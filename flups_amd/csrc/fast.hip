@@ -946,14 +946,14 @@ struct HybridZ {
     int M = 0, nx = 0, ny = 0, nz = 0, lda = 1, gtx = 8;
     bool real = false;       // r2c last direction (col_rz): the general path's Green's function, real columns
     bool xrow = false;       // r2c last direction along x (row_rz): real rows
-    void* twn = nullptr;     // row_rz: n-point table
+    const double* twn = nullptr;   // row_rz: n-point table
     double normfact = 1;
     const void* g = nullptr;     // real: the solver's spectral Green's function (not owned)
     bool f32 = false;            // FP32 stage arrays and Green's function (FP64 arithmetic)
     bool smooth = false;     // not a power of two: smooth_z
     bool pair = false, twod = false;
     void* green = nullptr;   // normfact * Re G, [y'][tile][kz'][gtx]
-    void* tw = nullptr;      // M-point table
+    const double* tw = nullptr;    // M-point table (row_rz: q-point); the tables are the solver's
     int rtx = 0;             // columns per block of the fused rotational pass (0: none)
     double* sym = nullptr;   // its derivative symbols: x, y, z
     size_t dev_bytes = 0;
@@ -1021,6 +1021,9 @@ HybridZ* make_hybrid_z(SolverImpl& s) {
         if (in.nf != 1 || sp.nf != 2 || !row_rz_len_ok(M) || sp.n[0] != M / 2 + 1 || in.n[0] > M || !s.dgreen_) return nullptr;
         for (int d = 1; d < nd; ++d)
             if (in.n[d] != sp.n[d]) return nullptr;
+        int pf = 1, q = 0;
+        split_pq(M / 2, pf, q);
+        const double *tw = s.twiddles(q), *twn = s.twiddles(M);
         auto* h = new HybridZ;
         h->f32 = f32;
         h->real = true;
@@ -1032,20 +1035,8 @@ HybridZ* make_hybrid_z(SolverImpl& s) {
         h->lda = s.lda_;
         h->normfact = s.normfact_;
         h->g = f32 ? (const void*)s.dgreen32_ : (const void*)s.dgreen_;
-        int pf = 1, q = 0;
-        split_pq(M / 2, pf, q);
-        const auto t = twiddle_table(q), tn = twiddle_table(M);
-        try {
-            HIP_CHECK(hipMalloc(&h->tw, t.size() * sizeof(double)));
-            HIP_CHECK(hipMemcpy(h->tw, t.data(), t.size() * sizeof(double), hipMemcpyHostToDevice));
-            HIP_CHECK(hipMalloc(&h->twn, tn.size() * sizeof(double)));
-            HIP_CHECK(hipMemcpy(h->twn, tn.data(), tn.size() * sizeof(double), hipMemcpyHostToDevice));
-        } catch (...) {
-            (void)hipFree(h->tw);
-            delete h;
-            throw;
-        }
-        h->dev_bytes = (t.size() + tn.size()) * sizeof(double);
+        h->tw = tw;
+        h->twn = twn;
         h->bytes = h->lda * 2.0 * (double)h->nx * h->ny * es + (double)h->ny * (M / 2 + 1) * 2 * es;
         return h;
     }
@@ -1057,6 +1048,7 @@ HybridZ* make_hybrid_z(SolverImpl& s) {
         const bool p2 = pow2_in(M, 32, 1024);
         const int smooth_tx = p2 ? 0 : smooth_z_tile(M, f32);
         if (!(p2 || smooth_tx) || sp.n[nd - 1] != M / 2 + 1 || in.n[nd - 1] > M || !s.dgreen_) return nullptr;
+        const double* tw = s.twiddles(M);
         auto* h = new HybridZ;
         h->smooth = !p2;
         h->gtx = smooth_tx;
@@ -1069,15 +1061,7 @@ HybridZ* make_hybrid_z(SolverImpl& s) {
         h->lda = s.lda_;
         h->normfact = s.normfact_;
         h->g = f32 ? (const void*)s.dgreen32_ : (const void*)s.dgreen_;
-        const auto t = twiddle_table(M);
-        try {
-            HIP_CHECK(hipMalloc(&h->tw, t.size() * sizeof(double)));
-            HIP_CHECK(hipMemcpy(h->tw, t.data(), t.size() * sizeof(double), hipMemcpyHostToDevice));
-        } catch (...) {
-            delete h;
-            throw;
-        }
-        h->dev_bytes = t.size() * sizeof(double);
+        h->tw = tw;
         // the field in and out, the Green's function's (M/2 + 1) rows of complex values
         h->bytes = h->lda * 2.0 * (double)h->nx * h->ny * h->nz * es + (double)h->nx * h->ny * (M / 2 + 1) * 2 * es;
         return h;
@@ -1085,9 +1069,11 @@ HybridZ* make_hybrid_z(SolverImpl& s) {
     const HybridC2C plan = plan_hybrid_c2c(s, f32);
     if (!plan.gtx) return nullptr;
     const int M = f.n_in[0];
+    const double* tw = s.twiddles(M);
     auto* h = new HybridZ;
     h->f32 = f32;
     h->M = M;
+    h->tw = tw;
     h->nx = in.n[0];
     h->ny = nd == 3 ? in.n[1] : 1;
     h->nz = in.n[nd - 1];
@@ -1106,10 +1092,6 @@ HybridZ* make_hybrid_z(SolverImpl& s) {
         hipLaunchKernelGGL(compress_green, dim3(4096), dim3(256), 0, s.stream_, s.dgreen_, f32 ? nullptr : (double*)h->green,
                            f32 ? (float*)h->green : nullptr, h->nx, h->ny, M, gy, gz, h->gtx, ntx, s.normfact_);
         HIP_CHECK(hipGetLastError());
-        const auto t = twiddle_table(M);
-        HIP_CHECK(hipMalloc(&h->tw, t.size() * sizeof(double)));
-        HIP_CHECK(hipMemcpy(h->tw, t.data(), t.size() * sizeof(double), hipMemcpyHostToDevice));
-        h->dev_bytes += t.size() * sizeof(double);
         if (h->rtx > 0) {   // derivative symbols of the rotational pass
             RotK rk{};
             for (int i = 0; i < nd; ++i) {
@@ -1126,11 +1108,9 @@ HybridZ* make_hybrid_z(SolverImpl& s) {
             HIP_CHECK(hipMemcpy(h->sym, t3.data(), t3.size() * sizeof(double), hipMemcpyHostToDevice));
             h->dev_bytes += t3.size() * sizeof(double);
         }
-        HIP_CHECK(hipStreamSynchronize(s.stream_));
     } catch (...) {
         (void)hipFree(h->sym);
         (void)hipFree(h->green);
-        (void)hipFree(h->tw);
         delete h;
         throw;
     }
@@ -1142,8 +1122,6 @@ HybridZ* make_hybrid_z(SolverImpl& s) {
 void destroy_hybrid_z(HybridZ* h) {
     if (!h) return;
     (void)hipFree(h->green);
-    (void)hipFree(h->tw);
-    (void)hipFree(h->twn);
     (void)hipFree(h->sym);
     delete h;
 }
@@ -1160,8 +1138,8 @@ void hybrid_z_t(const HybridZ* h, void* data, hipStream_t st) {
         A.f32 = std::is_same<S, float>::value;
         A.d = data;
         A.g = h->g;
-        A.tw = static_cast<const double*>(h->tw);
-        A.twn = static_cast<const double*>(h->twn);
+        A.tw = h->tw;
+        A.twn = h->twn;
         A.nin = h->nx;
         A.M = h->M;
         A.lda = h->lda;
@@ -1176,7 +1154,7 @@ void hybrid_z_t(const HybridZ* h, void* data, hipStream_t st) {
         A.f32 = std::is_same<S, float>::value;
         A.d = data;
         A.g = h->g;
-        A.tw = static_cast<const double*>(h->tw);
+        A.tw = h->tw;
         A.nx = h->nx;
         A.ny = h->ny;
         A.nin = h->nz;
@@ -1194,7 +1172,7 @@ void hybrid_z_t(const HybridZ* h, void* data, hipStream_t st) {
         A.f32 = std::is_same<S, float>::value;
         A.d = data;
         A.g = h->g;
-        A.tw = static_cast<const double*>(h->tw);
+        A.tw = h->tw;
         A.nx = h->nx;
         A.ny = h->ny;
         A.nin = h->nz;
@@ -1211,7 +1189,7 @@ void hybrid_z_t(const HybridZ* h, void* data, hipStream_t st) {
         A.f32 = std::is_same<S, float>::value;
         A.d = data;
         A.g = h->green;
-        A.tw = static_cast<const double*>(h->tw);
+        A.tw = h->tw;
         A.nx = h->nx;
         A.nother = h->ny;
         A.nin = h->nz;
@@ -1270,7 +1248,7 @@ void hybrid_z(const HybridZ* h, void* data, int type, hipStream_t st) {
         SmoothRotArgs A;
         A.d = data;
         A.g = h->green;
-        A.tw = static_cast<const double*>(h->tw);
+        A.tw = h->tw;
         A.sym = h->sym;
         A.off[1] = h->nx;
         A.off[2] = h->nx + h->ny;

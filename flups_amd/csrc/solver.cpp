@@ -300,10 +300,21 @@ const double* SolverImpl::twiddles(int M) {
         t[2 * i] = (double)cosl(a);
         t[2 * i + 1] = (double)sinl(a);
     }
+    return tw_[M] = upload(std::move(t));
+}
+
+// a table in device memory. Set-up queues its copy on the stream, behind nothing but set-up's own kernels, and waits once at
+// its end (a blocking copy each: about 30 us of the 40 that a table takes)
+double* SolverImpl::upload(std::vector<double> t) {
     double* d = nullptr;
-    HIP_CHECK(hipMalloc(&d, t.size() * sizeof(double)));
-    HIP_CHECK(hipMemcpy(d, t.data(), t.size() * sizeof(double), hipMemcpyHostToDevice));
-    tw_[M] = d;
+    const size_t bytes = t.size() * sizeof(double);
+    HIP_CHECK(hipMalloc(&d, bytes));
+    if (setup_done_) {
+        HIP_CHECK(hipMemcpy(d, t.data(), bytes, hipMemcpyHostToDevice));
+        return d;
+    }
+    pending_.push_back(std::move(t));   // the source lives until set-up's last wait
+    HIP_CHECK(hipMemcpyAsync(d, pending_.back().data(), bytes, hipMemcpyHostToDevice, stream_));
     return d;
 }
 
@@ -312,12 +323,7 @@ const double* SolverImpl::r2r_table(int kind, int n) {
     auto it = r2r_tab_.find(key);
     if (it != r2r_tab_.end()) return it->second;
     FLUPS_REQUIRE(!frozen_, "real-to-real table (kind %d, n %d) missing in a solve that may not allocate", kind, n);
-    const auto t = row_r2r_table(kind, n);
-    double* d = nullptr;
-    HIP_CHECK(hipMalloc(&d, t.size() * sizeof(double)));
-    HIP_CHECK(hipMemcpy(d, t.data(), t.size() * sizeof(double), hipMemcpyHostToDevice));
-    r2r_tab_[key] = d;
-    return d;
+    return r2r_tab_[key] = upload(row_r2r_table(kind, n));
 }
 
 void SolverImpl::plan_fft(PassDesc& P, int M) {
@@ -331,7 +337,6 @@ void SolverImpl::plan_fft(PassDesc& P, int M) {
         while (m % p == 0) { P.rad[P.nst++] = p; m /= p; }
     }
     FLUPS_REQUIRE(P.nst <= 16, "transform length %d has too many factors", M);
-    P.tw = twiddles(M);
 }
 
 // Arrays larger than half the 256 MB Infinity Cache are read or written with non-temporal
@@ -462,6 +467,7 @@ PassDesc SolverImpl::pass_desc(const DirPlan& p, int comp, bool forward, const V
     // contiguous real-to-complex pencils, and the same shapes at the other lengths with factors 2, 3, 5, 7: run-time
     // mixed radix
     if (!std::getenv("FLUPS_GENERIC_PASS") && smooth_pass(P)) return P;
+    P.tw = twiddles(M);
     P.alias = generic_alias(P) ? 1 : 0;
     const size_t per_pen = generic_lds_bytes(P, 1);
     FLUPS_REQUIRE(per_pen <= lds_budget_, "pencil of %d elements (transform length %d) does not fit the general path's LDS",
@@ -798,6 +804,7 @@ void SolverImpl::setup() {
     }
     scratch_init();   // this device's static scratch address, for flups_solve_noalloc
     HIP_CHECK(hipStreamSynchronize(stream_));
+    pending_.clear();
     setup_done_ = true;
     if (prof_) prof_->add("setup", std::chrono::duration<double>(std::chrono::steady_clock::now() - t_setup).count(), 0.0);
 }
@@ -1022,6 +1029,10 @@ void SolverImpl::warm_tables() {
     const View u = user_view(static_cast<double*>(dstage_[0]));
     std::vector<int> fk(2 * ndim_, 0);
     for (int ip = 0; ip < ndim_; ++ip) {
+        if (fused_only() && ip == ndim_ - 1) {   // no solve runs its passes
+            fk[ip] = fk[ndim_ + ip] = -2;
+            continue;
+        }
         const View prev = (ip == 0) ? u : dense_view(dstage_[ip - 1], stage_[ip - 1], ses_);
         const View cur = dense_view(dstage_[ip], stage_[ip], ses_);
         for (int c = 0; c < lda_; ++c) {

@@ -140,6 +140,8 @@ class SolverImpl {
     std::map<int, double*> tw_;
     std::map<std::pair<int, int>, double*> r2r_tab_;   // (kind, n) -> pre / post twiddles of the row r2r kernel
     const double* r2r_table(int kind, int n);
+    double* upload(std::vector<double> t);
+    std::vector<std::vector<double>> pending_;   // set-up's queued copies: their sources
     void* dstage_[3] = {nullptr, nullptr, nullptr};   // general path stage arrays: double, or float (gf32_)
     double* dgreen_ = nullptr;
     float* dgreen32_ = nullptr;   // FP32 copy of the Green's function (gf32_)
