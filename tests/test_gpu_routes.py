@@ -11,10 +11,24 @@ except Exception:   # pragma: no cover
     torch = None
 
 import flups_amd as fl
+from tests.test_gpu_parity import TOL, rel_err
+from tests.test_gpu_rot import GENERAL, field as rot_field, solve as rot_solve
 
 pytestmark = pytest.mark.gpu
 
-U = 4
+O, P, U = 1, 3, 4
+# columns of 1120 points (three components and one column take 53760 of 54272 bytes), 1024, and 945 of a full column
+LONG = {
+    "z-560": ((20, 18, 560), [[U, U]] * 3, 1, 1),
+    "z-512": ((20, 18, 512), [[P, P], [P, P], [U, U]], 1, 2),
+    "periodic-z-945": ((18, 20, 945), [[P, P]] * 3, 1, 1),
+}
+# 1350 points: no tile fits; walls: their derivative is no multiplication by i K
+NOT_FUSED = {
+    "z-675": GENERAL["z-675"],
+    "walls-z-40": ((24, 20, 40), [[O, O], [P, P], [U, U]], 1, 1),
+}
+ROT = {**GENERAL, **LONG, **NOT_FUSED}
 
 
 class KernelNode(ctypes.Structure):   # hipKernelNodeParams
@@ -74,3 +88,28 @@ def test_schedule_is_what_runs(monkeypatch, nglob):
     slabs = run({"FLUPS_SLAB_MB": 0.25, "FLUPS_ZSCHED": 20})[0]
     assert len(slabs) > 5
     assert sum(slabs[2:-1:3]) == default[2], (slabs, default)
+
+
+@pytest.mark.parametrize("fp32", [False, True], ids=["fp64", "fp32"])
+@pytest.mark.parametrize("name", ROT)
+def test_rotational_last_direction_is_fused(name, fp32):
+    """the curl runs inside the last direction (two passes, the fused one, two passes) wherever its columns fit a block, and
+    as three passes, the multiply and three passes where they do not"""
+    nglob, bc, center, odiff = ROT[name]
+    h = [1.0 / (max(nglob) - (1 - center))] * 3
+    r = fl.ServeRequest.make(nglob, bc, h, [h[0] * (m - (1 - center)) for m in nglob], green=0, lda=3, center=center, fp32=fp32,
+                             solver_type=1, order_diff=odiff)
+    b = fl.Batch([r], [fl.DeviceArray(r.shape())], [fl.DeviceArray(r.shape())])
+    n = b.launches(False)
+    assert n >= 7 if name in NOT_FUSED else n == 5, n
+
+
+@pytest.mark.parametrize("fp32", [False, True], ids=["fp64", "fp32"])
+@pytest.mark.parametrize("name", LONG)
+def test_rotational_columns_of_one_per_block(name, fp32):
+    """the longest columns that fit: one per block"""
+    nglob, bc, center, odiff = LONG[name]
+    got, path, ora = rot_solve(nglob, bc, center, odiff, rot_field(nglob), fp32)
+    assert path == (5 if fp32 else 3)
+    e2, ei = rel_err(got, ora)
+    assert max(e2, ei) <= (1e-5 if fp32 else TOL), (e2, ei)
