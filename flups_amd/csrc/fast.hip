@@ -46,7 +46,7 @@
 namespace flups {
 
 template <typename R>
-void launch_z_rot(int M, const ColArgs& a, const RotK& rk, hipStream_t st);   // zrot.hip
+void launch_z_rot(int M, const ColArgs& a, const RotSym& rk, hipStream_t st);   // zrot.hip
 
 namespace {
 
@@ -229,6 +229,12 @@ struct z_fused {
             }
         }
     }
+};
+
+// wave numbers of the rotational pass
+struct RotK {
+    double kfact[3], h[3], symstart[3];
+    int order;   // 1 spectral, 2 / 4 / 6 centred differences
 };
 
 // derivative symbol of mode idx along d: symmetrised index (mirrored half negative),
@@ -445,6 +451,7 @@ struct FastPlan {
     size_t nt_bytes = (size_t)128 << 20;   // stage arrays from this size on: non-temporal accesses (FLUPS_NT_MB)
     int gtx = 0;             // x tile width of the compressed Green's layout
     RotK rot{};              // wave-number data of the rotational pass
+    RotSym rsym{};           // its derivative symbols on the device
     void* s0 = nullptr;     // (ldx, N1, N2) complex, FP64 or FP32
     void* s1 = nullptr;     // one x slab of the y-transformed field: (ldxs, M1, N2) complex, z stride zs
     long long ldxs = 0;     // S1 row length: the widest slab
@@ -618,7 +625,7 @@ void build_fast_plan(SolverImpl& s, FastPlan* f, size_t es, int align) {
         const int nsym[3] = {f->nx, f->M[1], f->M[2]};
         std::vector<double> t;
         for (int d = 0; d < 3; ++d) {
-            f->rot.off[d] = (int)t.size();
+            f->rsym.off[d] = (int)t.size();
             for (int i = 0; i < nsym[d]; ++i) t.push_back(rot_symbol(f->rot, d, i));
         }
         void* d = nullptr;
@@ -632,7 +639,7 @@ void build_fast_plan(SolverImpl& s, FastPlan* f, size_t es, int align) {
         }
         f->owned.push_back(d);
         f->dev_bytes += t.size() * (f->fp32 ? sizeof(float) : sizeof(double));
-        f->rot.sym = d;
+        f->rsym.sym = d;
     }
     f->ev.assign(3 + 3 * (f->slab.size() - 1), nullptr);
     for (auto& e : f->ev) HIP_CHECK(hipEventCreate(&e));
@@ -838,7 +845,6 @@ void run_fast(FastPlan* f, void* s0, void* s1, const double* rhs, double* field,
         z.nout = N2;
         z.gy = M1 / 2 + 1;
         z.gmy = M1;
-        z.gmz = M2;
         z.comp_src = c1;
         z.comp_dst = c1;
         z.xcd = (f->zsched >> 4) & 1;
@@ -853,7 +859,7 @@ void run_fast(FastPlan* f, void* s0, void* s1, const double* rhs, double* field,
             // rotational pass: all three components per block
             FLUPS_REQUIRE(f->lda == 3, "the rotational solve needs lda = 3");
             z.gtx = f->gtx;
-            launch_z_rot<R>(M2, z, f->rot, st);
+            launch_z_rot<R>(M2, z, f->rsym, st);
         } else {
             col_dispatch<R, TX, true, true>(M2, z, f->lda, f->zsched, st);
         }
@@ -1219,7 +1225,6 @@ void hybrid_z_t(const HybridZ* h, void* data, hipStream_t st) {
     z.nout = h->nz;
     z.gy = h->pair ? h->ny / 2 + 1 : h->ny;
     z.gmy = h->pair ? h->ny : 0;
-    z.gmz = h->M;
     z.comp_src = (long long)h->nx * h->ny * h->nz;
     z.comp_dst = z.comp_src;
     z.xcd = 1;

@@ -17,9 +17,8 @@ struct ColArgs {
     long long s_other_src, s_other_dst;   // stride of the other (batch) dimension
     int nother;
     int nin, nout;       // valid input rows, rows to store
-    int gy, gmy, gmz;    // z_fused: ky' extent, M1 (for ky' = min(y, M1-y)), M2
-    int cstride_src, cstride_dst;   // component strides in complex elements (low 32 bits)
-    long long comp_src, comp_dst;
+    int gy, gmy;         // z_fused: ky' extent, M1 (for ky' = min(y, M1-y))
+    long long comp_src, comp_dst;   // component strides in complex elements
     int rev;             // 1: blocks walk the batch from its last entry
     int xcd;             // z_fused: 1 = XCD-grouped block numbering
     int nopair;          // z_fused: 1 = the other dim has no mirror rows (one row per block, G stored per row)
@@ -29,12 +28,10 @@ struct ColArgs {
     int nt;              // col_fft forward: 1 = non-temporal stores
 };
 
-// wave numbers of the rotational z pass
-struct RotK {
-    double kfact[3], h[3], symstart[3];
-    int order;          // 1 spectral, 2 / 4 / 6 centred differences
-    const void* sym;    // derivative symbols by mode index: x (nx), then y (M1), then z (M2), type R
-    int off[3];         // start of each direction's table
+// derivative symbols of the rotational z pass by mode index: x (nx), y (M1), z (M2), type R, from off[d] on
+struct RotSym {
+    const void* sym;
+    int off[3];
 };
 
 }  // namespace flups

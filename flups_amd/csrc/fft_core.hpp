@@ -247,18 +247,17 @@ __device__ __forceinline__ void column_fft(C2<R>* v, C2<R>* lds, int j, const C2
     }
 }
 
-// Column FFT of length H = P Q (P = 1, 3, 5 or 7; Q a power of two, at least 8) held by
+// Column FFT of length H = P Q (P = 1 or 3; Q a power of two, at least 8) held by
 // T = Q/8 threads with 8P values each: on entry v[i] = x[j + i T], on exit v[i] = X[j + i T]
 // (i < 8P). For P > 1 (Cooley-Tukey with n = Q n1 + n2, k = k1 + P k2): the P-point DFTs
 // over n1 (a thread holds every n1 of its n2 = j + i T), the twiddles w_H^(n2 k1), the P
 // Q-point column FFTs over n2 one after the other on the same LDS, and an LDS exchange back
 // to the natural order. twq: Q-point table; twh[e * hs] = exp(-2 pi i e / H). The whole block
 // calls this together; it ends with LDS reads (sync before the next LDS write).
-template <typename R, int P, int Q, bool FWD, int ES, bool HIN = false, bool LTW = false>
+template <typename R, int P, int Q, bool FWD, int ES, bool HIN = false>
 __device__ __forceinline__ void column_fft_pq(C2<R>* v, C2<R>* lds, int j, const C2<R>* twq, const C2<R>* twh, int hs) {
-    static_assert(P == 1 || !LTW, "LDS twiddles for powers of two only");
     if constexpr (P == 1) {
-        column_fft<R, Q, FWD, ES, HIN, LTW>(v, lds, j, twq);
+        column_fft<R, Q, FWD, ES, HIN>(v, lds, j, twq);
     } else {
         constexpr int T = Q / 8;
         C2<R> wp[P];   // w_P^m = w_H^(m Q)

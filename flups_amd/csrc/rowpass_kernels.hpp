@@ -304,7 +304,7 @@ struct pen_r2r {
     }
 };
 
-// M = PF Q: PF = 1 (a power of two) or 3, 5 (8 PF values per thread, column_fft_pq)
+// M = PF Q: PF = 1 (a power of two) or 3 (8 PF values per thread, column_fft_pq)
 template <int PF, int Q, int TX, bool FWD, typename TI, typename TO>
 struct col_real {
     using Args = PassDesc;

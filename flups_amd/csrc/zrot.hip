@@ -17,7 +17,7 @@ namespace {
 
 struct ZRotArgs {
     ColArgs a;
-    RotK rk;
+    RotSym rk;
 };
 
 // A block transforms one row of TX columns (64-byte rows of HBM) of the three components at a time:
@@ -145,7 +145,7 @@ struct z_rot {
 // Blocks that fill the chip: 256 CUs, kWaves waves on each of their four SIMDs. TX: 64-byte rows, but
 // at least a whole wave a block, and at most 512 threads.
 template <typename R, int M>
-void launch(const ColArgs& a, const RotK& rk, hipStream_t st) {
+void launch(const ColArgs& a, const RotSym& rk, hipStream_t st) {
     constexpr int W = 64 / (int)sizeof(C2<R>);
     constexpr int TX = M <= 64 ? std::max(W, 512 / M) : M == 1024 ? 4 : W;
     constexpr int full = 256 * (sizeof(R) == 8 ? 8 : 16) * 64 / (TX * M / 8);
@@ -160,7 +160,7 @@ void launch(const ColArgs& a, const RotK& rk, hipStream_t st) {
 }  // namespace
 
 template <typename R>
-void launch_z_rot(int M, const ColArgs& a, const RotK& rk, hipStream_t st) {
+void launch_z_rot(int M, const ColArgs& a, const RotSym& rk, hipStream_t st) {
     switch (M) {
         case 32: launch<R, 32>(a, rk, st); break;
         case 64: launch<R, 64>(a, rk, st); break;
@@ -171,7 +171,7 @@ void launch_z_rot(int M, const ColArgs& a, const RotK& rk, hipStream_t st) {
         default: fail("unsupported column length %d", M);
     }
 }
-template void launch_z_rot<double>(int, const ColArgs&, const RotK&, hipStream_t);
-template void launch_z_rot<float>(int, const ColArgs&, const RotK&, hipStream_t);
+template void launch_z_rot<double>(int, const ColArgs&, const RotSym&, hipStream_t);
+template void launch_z_rot<float>(int, const ColArgs&, const RotSym&, hipStream_t);
 
 }  // namespace flups
