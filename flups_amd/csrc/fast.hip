@@ -552,7 +552,7 @@ FastPlan* make_fast_plan(SolverImpl& s) {
     if (f->zsched < 0 || f->zsched > 63 || (f->zsched & 3) == 3 || ((f->zsched & 8) && (f->zsched & 7))) {
         delete f;
         fail("FLUPS_ZSCHED: bits 0-1 schedule (0, 1, 2), bit 2 half-width tiles, bit 3 quarter-width tiles (schedule 0), "
-             "bit 4 XCD-grouped blocks, bit 5 mirror rows in neighbouring blocks");
+             "bit 4 XCD-grouped blocks, bit 5 the row pairing that the problem's size does not take by itself");
     }
     try {
         build_fast_plan(s, f, es, align);
@@ -561,6 +561,17 @@ FastPlan* make_fast_plan(SolverImpl& s) {
         throw;
     }
     return f;
+}
+
+// The two rows of a mirror pair in one block (one read of G's slice) or in neighbouring blocks: apart where the pairs are
+// less than three rounds of the chip's waves (16 on each of 256 CUs), and the other way round with bit 5 of the
+// schedule. A function of the whole problem and the schedule (an x slab does as the field does). Solves, FP64, in one
+// block -> apart, us: open 32^3 26.4 -> 25.1, 64^3 40.7 -> 40.0, 64 x 64 x 256 65.5 -> 62.6, 128^3 100.1 -> 98.4;
+// three components of 128^3 281.6 -> 285.7, 128 x 128 x 256 195 -> 197. Schedules 1 and 2 were not measured: in one block
+static bool rows_apart(const FastPlan* f) {
+    const double waves = (double)f->nx * (f->M[1] / 2 + 1) * f->lda * f->M[2] / 512;
+    const bool small = (f->zsched & 3) == 0 && waves < 3 * 16 * 256;
+    return small != ((f->zsched & 32) != 0);
 }
 
 // x tile width of the z kernel for the plan's schedule: half the stage tile for
@@ -848,11 +859,7 @@ void run_fast(FastPlan* f, void* s0, void* s1, const double* rhs, double* field,
         z.comp_src = c1;
         z.comp_dst = c1;
         z.xcd = (f->zsched >> 4) & 1;
-        // the two rows of a mirror pair in one block (one read of G's slice); bit 5: in neighbouring blocks. What
-        // the schedule says and nothing else: the neighbours are faster where the field is small (open 32^3 26.4 -> 25.1,
-        // 64^3 40.7 -> 40.0, 128^3 100.1 -> 98.4 us; three components of 128^3 281.6 -> 285.7) and slower
-        // from 128 x 128 x 256 on (195 -> 197)
-        z.nopair = (f->zsched & 32) ? 2 : 0;
+        z.nopair = rows_apart(f) ? 2 : 0;
         z.x0 = x0;
         z.gntx = (f->nx + f->gtx - 1) / f->gtx;
         if (type == 1) {

@@ -21,7 +21,8 @@ struct ColArgs {
     long long comp_src, comp_dst;   // component strides in complex elements
     int rev;             // 1: blocks walk the batch from its last entry
     int xcd;             // z_fused: 1 = XCD-grouped block numbering
-    int nopair;          // z_fused: 1 = the other dim has no mirror rows (one row per block, G stored per row)
+    int nopair;          // z_fused: 1 = the other dim has no mirror rows (one row per block, G stored per row); 2 = the two
+                         // rows of a pair in neighbouring blocks
     int x0;              // z_fused / z_rot: spectral x index of column 0 (slab offset, a multiple of TX)
     int gntx;            // z_fused / z_rot: x tiles of one ky' row of the compressed G
     int gtx;             // z_rot: tile width of the compressed G
