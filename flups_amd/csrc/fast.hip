@@ -938,13 +938,18 @@ size_t fast_device_bytes(const FastPlan* f) { return f->dev_bytes; }
 
 // ---------------------------------------------------------------------------
 // Last direction of the general path fused with the multiply: when the final
-// forward transform is a c2c along z (unbounded or cell-centred periodic) of a
-// power-of-two length, the forward z FFT, the Green's multiply and the inverse
-// z FFT run as one z_fused launch in place on the stage array before it (the
-// general passes do the other directions). The other dim (y) may be a
-// half-spectrum (r2c) or real-to-real direction: rows are not paired then.
-// 2-D problems fuse their last direction (y) the same way, as a 3-D field with
-// one row (columns up to 2048 long, two columns per block).
+// forward transform is unbounded or cell-centred periodic, the forward FFT, the
+// Green's multiply and the inverse FFT run as one launch in place on the stage
+// array before it (the general passes do the other directions).
+//  * c2c along z: z_fused for powers of two, smooth_z for the other lengths with
+//    factors 2, 3, 5, 7; smooth_rot takes the curl of three components as well.
+//    The other dim (y) may be a half-spectrum (r2c) or real-to-real direction: rows
+//    are not paired then. 2-D problems fuse their last direction (y) the same way, as
+//    a 3-D field with one row (columns up to 2048 long, two columns per block). Their
+//    G is a compressed copy, normfact folded in (1/8 of the general path's where rows
+//    pair, else 1/4); the last stage array is not allocated in its place.
+//  * r2c along z (every other direction real-to-real): col_rz and smooth_rz, pairs of
+//    real columns; along x: row_rz. They read G from the general path's layout.
 void launch_col_rz(const RzArgs& A, hipStream_t s);   // rowpass.hip
 void launch_row_rz(const RzArgs& A, hipStream_t s);
 bool row_rz_len_ok(int M);

@@ -10,9 +10,12 @@
 //                strided one), pre- and post-maps from tables (smooth_pen.hpp).
 // Before, these lengths ran on the generic kernel (up to five radix 2-7 stages over LDS, sines and
 // cosines computed in its pre- and post-maps, 2n-point extensions for r2r) with a separate multiply
-// sweep: 200 x 144 x 100 open 6 x 262 + 80 us, now 48 (x) + 51 (y) + 131 (fused z) + 51 + 48 us, the
-// solve 1589 -> 331 us; 240 x 100 x 180 channel 1009 -> 211 us (MI355X, FP64). The passes move their
-// minimum bytes at 1.4-2.2 TB/s: bound by the latency of a block's load - stages - store chain.
+// sweep: 200 x 144 x 100 open 6 x 262 + 80 us, now 28 (x) + 33 (y) + 85 (fused z) + 33 + 28 us, the
+// solve 1589 -> 215 us; 240 x 100 x 180 channel 1009 -> 152 us (MI355X, FP64). The passes move their
+// minimum bytes at 2.1-4.2 TB/s. Counters of those two problems: 2.2 to 5.5 waves per SIMD resident, 39-63 % of
+// their cycles waiting on memory or a barrier, VALU busy 32-62 %, LDS bank conflicts 9-35 % of a CU's cycles:
+// the latency of a block's load - stages - store chain, but for the fused z of three stages (200 points: VALU
+// 62 %, conflicts 35 %).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -35,7 +38,8 @@ namespace {
 // 128 they spilled 20 to 40 (120^3 open 140 -> 126 us, 240^3 periodic 349 -> 316), and a block of
 // 64 threads and 12 KB of LDS reaches no fourth wave. Otherwise up to 10 in 80 registers, six waves: with three
 // stages the barriers between them want the waves (200 x 144 x 100 open: fused z 131 us with every
-// radix in one kernel, 84 us so; five waves 193 -> 199, seven 196, eight 225 us the solve)
+// radix in one kernel, 84 us so; five waves 193 -> 199, seven 196, eight 225 us the solve), although the
+// narrow ones of smooth_col and smooth_z spill 20 to 36 bytes at six
 template <bool WIDE, typename TI, typename TO>
 struct smooth_col {
     using Args = PassDesc;
@@ -200,7 +204,8 @@ struct smooth_z {
 // An r2c last direction: two neighbouring real columns a, b as one complex column a + i b, whose product
 // spectrum is Z'[k] = Ga/2 (Z[k] + conj Z[M-k]) + Gb/2 (Z[k] - conj Z[M-k]) (G real and even in kz). The mirrored value
 // lies with another thread: the forward spectrum passes through LDS between the transforms.
-// 129 x 161 x 97 node-centred walls, MI355X: r2c 22, multiply 15 and c2r 23 us before, 27 us now.
+// 129 x 161 x 97 node-centred walls, MI355X: r2c 22, multiply 15 and c2r 23 us before, 27 us now. Two sets of G beside the
+// values: four waves (128 registers, nothing spilled), three for the wide radices (168, 40 bytes spilled).
 template <bool WIDE, typename ST>
 struct smooth_rz {
     using Args = SmoothRzArgs;

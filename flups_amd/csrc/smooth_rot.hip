@@ -8,7 +8,8 @@
 // component's LDS reads and its writes lies one barrier, which also orders the component before it, so a
 // stage costs three barriers for three transforms. The last forward stage, the curl and the
 // first inverse stage (the same radix) touch a thread's own LDS slots only. 160^3 layer, FP32
-// storage, MI355X: 3 x 30 + 70 + 3 x 30 us -> 149 us, the solve 556 -> 450 us.
+// storage, MI355X: 3 x 30 + 70 + 3 x 30 us -> 145 us. 50 MB in, 50 MB out and 4 MB of G, 0.7 TB/s: bound inside the
+// block (counters: 2.3 waves per SIMD resident, VALU busy 40 %, LDS bank conflicts 38 % of a CU's cycles).
 #include <hip/hip_runtime.h>
 
 #include "core.hpp"
@@ -163,7 +164,11 @@ struct smooth_rot {
 };
 
 // bytes of one block: three blocks share a CU's 160 KB. Narrower tiles rather than two larger blocks: 80^3 open FP32 175 ->
-// 161 us (8 -> 4 columns), 160^3 open 1103 -> 1093 (4 -> 2), 160^3 layer 365 -> 361; 32 KB: batch 1548 -> 1635
+// 161 us (8 -> 4 columns), 160^3 open 1103 -> 1093 (4 -> 2), 160^3 layer 365 -> 361; 32 KB: batch 1548 -> 1635.
+// Two columns from 288 points on and one from 567 on (16-byte rows, 8 in FP32) still beat three passes, the multiply
+// and three passes by the same kernels, up to the longest column that fits (solves, us, separate -> fused, FP64 / FP32):
+// 96 x 96 periodic with 512 points 416 -> 343 / 344 -> 310, 576: 480 -> 437 / 368 -> 361, 640: 550 -> 505 / 417 -> 382, 1024: 958 ->
+// 821 / 755 -> 619, 1120: 1256 -> 1017 / 970 -> 743; 48 x 48 open with 450 points 224 -> 165, 640: 284 -> 219, 1120: 723 -> 549
 constexpr size_t kRotLds = 54272;
 
 // Radices up to 10 where the tile's LDS limits the waves: 112^3 open 389 -> 367 us, layer 157 -> 143, 96^3 layer 107 ->
