@@ -123,6 +123,7 @@ struct PassDesc {
     int nt = 0;             // row r2r kernel: its vector accesses are non-temporal (both arrays 128 MiB or more)
     const double* aux = nullptr;   // fast kernels: pre / post twiddle table
     SmoothPlan sm;          // M > 0: kernels of smooth.hip, their stages (sm.T threads per pencil, ppb pencils per block)
+    int comps = 1;                      // components of the pass (the size that a choice of kernel looks at)
     int lda = 1;                        // components of the launch, src_c / dst_c reals apart
     long long src_c = 0, dst_c = 0;
     template <typename T>

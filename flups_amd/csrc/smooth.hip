@@ -19,6 +19,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <array>
 #include <cstdint>
 #include <map>
 #include <mutex>
@@ -341,12 +342,12 @@ int col_tile(int M, int T, bool f32) {
 // fewest stages, then radices up to 10 (the kernels with fewer registers), then fewest threads (the
 // largest smallest radix); radices ascending, so that every thread takes part in the first stage and in
 // the last one of a fused inverse, the ones that meet HBM
-static bool search_plan(int M, int maxrad, SmoothPlan& p) {
+static bool search_plan(int M, int maxrad, int minst, SmoothPlan& p) {
     static const int rads[13] = {2, 3, 4, 5, 6, 7, 8, 9, 10, 12, 14, 15, 16};
     std::vector<int> cur, best;
     auto search = [&](auto&& self, int m, int lo) -> void {
         if (m == 1) {
-            if (cur.size() < 2) return;
+            if ((int)cur.size() < minst) return;
             const bool low = cur.back() <= 10, blow = !best.empty() && best.back() <= 10;
             if (best.empty() || cur.size() < best.size() ||
                 (cur.size() == best.size() && (low != blow ? low : cur[0] > best[0])))
@@ -386,24 +387,41 @@ static bool search_plan(int M, int maxrad, SmoothPlan& p) {
     }
     return p.T <= kSmoothThreads;
 }
-// every pass of every solve asks: the answers (a function of M and of the largest radix alone, a few thousand
-// at most) are kept
-bool smooth_plan_upto(int M, int maxrad, SmoothPlan& p) {
+// every pass of every solve asks: the answers (a function of M, of the largest radix and of the fewest stages
+// alone, a few thousand at most) are kept
+bool smooth_plan_upto(int M, int maxrad, SmoothPlan& p, int minst) {
     if (M < 16 || M > 2048) return false;
     static std::mutex mu;
-    static std::map<std::pair<int, int>, SmoothPlan> known;   // M = 0: no plan
+    static std::map<std::array<int, 3>, SmoothPlan> known;   // M = 0: no plan
     std::lock_guard<std::mutex> lk(mu);
-    const auto key = std::make_pair(M, maxrad);
+    const std::array<int, 3> key = {M, maxrad, minst};
     auto it = known.find(key);
     if (it == known.end()) {
         SmoothPlan q;
-        if (!search_plan(M, maxrad, q)) q = SmoothPlan();
+        if (!search_plan(M, maxrad, minst, q)) q = SmoothPlan();
         it = known.emplace(key, q).first;
     }
     p = it->second;
     return p.M == M;
 }
-bool smooth_plan(int M, SmoothPlan& p) { return smooth_plan_upto(M, 16, p); }
+bool smooth_plan(int M, SmoothPlan& p) { return smooth_plan_upto(M, 16, p, 2); }
+
+// Pencils: fewest stages, but three of radix 10 at most in the place of two where the two leave the chip short of waves: a stage
+// of radix R has M / R threads, so three stages have twice to four times the waves for one more trip through LDS. The
+// line lies at 1152 waves (256 CUs of four SIMDs), at 512 where the three begin with radix 2 (twice the threads of any
+// other stage). Measured on whole solves (FP64, two stages -> three) at 40 lengths from 20 to 256: up to 1024 waves
+// 0-30 % faster (32 x 320 x 32 walls in x and y, h = 160: 17-20 %), at 1152 from 5 % slower to 8 % faster, from 1500 up to
+// 20 % slower (h = 100); beginning with 2, up to 640 waves 1-20 % faster, at 1024 from 4 % slower to 7 % faster.
+// Rows from 224 points on, whose two radices are both 14 or more, take three always (rows of 512 periodic points: 10-18 %
+// faster up to the largest fields; columns of that length 4 % slower to 14 % faster, left at the line).
+static bool pen_plan(const PassDesc& P, int h, bool col, SmoothPlan& p) {
+    if (!smooth_plan(h, p)) return false;
+    SmoothPlan q;
+    if (p.nst != 2 || !smooth_plan_upto(h, 10, q, 3)) return true;
+    const long long waves = (long long)P.n1 * P.n2 * P.comps * p.T / 64;
+    if ((!col && h >= 224) || waves <= (q.rad[0] == 2 ? 512 : 1152)) p = q;
+    return true;
+}
 
 bool smooth_col_tile(PassDesc& P, int n) {
     if (!smooth_plan(n, P.sm)) return false;
@@ -418,7 +436,7 @@ void launch_smooth_col(const PassDesc& P, hipStream_t s) {
 // about 128 threads a block of contiguous pencils (64: 48, 128: 36, 256: 37, 512: 45 us a pass of 200 reals),
 // 16 neighbours of strided ones (128-byte rows; 4: 67, 8: 56, 16: 48, 32: 67 us a pass of 100 reals)
 bool smooth_pen_tile(PassDesc& P, int h, bool col) {
-    if (!smooth_plan(h, P.sm)) return false;
+    if (!pen_plan(P, h, col, P.sm)) return false;
     if (col) {
         P.ppb = fit_tile(16, P.sm.T, [&](int np) { return pen_lds(P, true, np); });
         return P.ppb > 0;

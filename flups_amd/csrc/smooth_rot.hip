@@ -19,7 +19,7 @@
 
 namespace flups {
 
-bool smooth_plan_upto(int M, int maxrad, SmoothPlan& p);   // smooth.hip
+bool smooth_plan_upto(int M, int maxrad, SmoothPlan& p, int minst);   // smooth.hip
 
 namespace {
 
@@ -174,7 +174,7 @@ constexpr size_t kRotLds = 54272;
 // Radices up to 10 where the tile's LDS limits the waves: 112^3 open 389 -> 367 us, layer 157 -> 143, 96^3 layer 107 ->
 // 95, 32 mixed problems 1555 -> 1525 against up to 16 (two stages, but three blocks of 64 threads a
 // CU); up to 8 the same within 1 %, up to 6 slower (80^3 open 153 -> 254). Every length that fits has such a plan.
-bool rot_plan(int M, SmoothPlan& p) { return smooth_plan_upto(M, 10, p); }
+bool rot_plan(int M, SmoothPlan& p) { return smooth_plan_upto(M, 10, p, 2); }
 
 }  // namespace
 

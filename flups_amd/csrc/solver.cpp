@@ -351,6 +351,7 @@ PassDesc SolverImpl::pass_desc(const DirPlan& p, int comp, bool forward, const V
                                const Shape& tout, int gshift, int sshift) {
     PassDesc P;
     P.d = p.dim;
+    P.comps = p.lda;
     P.sign = p.sign;
     P.n_out_plan = p.n_out;
     P.post = p.post[comp];

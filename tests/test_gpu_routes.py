@@ -36,8 +36,8 @@ class KernelNode(ctypes.Structure):   # hipKernelNodeParams
                 ("params", ctypes.c_void_p), ("shared", ctypes.c_uint)]
 
 
-def grids(solver, nglob):
-    """x extents of the grids of one solve's launches, in order: a captured flups_solve_noalloc"""
+def launches(solver, nglob):
+    """(grid, block) x extents of one solve's launches, in order: a captured flups_solve_noalloc"""
     hip = fl.lib()   # the HIP runtime that the library is linked with
     stream = fl.Stream()
     solver.set_stream(stream)
@@ -57,7 +57,7 @@ def grids(solver, nglob):
     for node in nodes:
         k = KernelNode()
         assert hip.hipGraphKernelNodeGetParams(ctypes.c_void_p(node), ctypes.byref(k)) == 0
-        out.append(int(k.grid[0]))
+        out.append((int(k.grid[0]), int(k.block[0])))
     assert hip.hipGraphDestroy(graph) == 0
     solver.set_stream(None)
     return out
@@ -81,7 +81,7 @@ def test_schedule_is_what_runs(monkeypatch, nglob, small):
         assert s.path == (1 if small else 2)
         s.solve(out, rhs)
         results.append(out.numpy())
-        return grids(s, nglob), s.schedule
+        return [g for g, _ in launches(s, nglob)], s.schedule
 
     results = []
     rhs = fl.DeviceArray.from_numpy(np.random.default_rng(2).normal(size=(1,) + nglob[::-1]))
