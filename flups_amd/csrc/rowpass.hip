@@ -5,6 +5,8 @@
 
 namespace flups {
 
+bool smooth_pen_wide(const PassDesc& P, int h);   // smooth.hip
+
 FLUPS_ROWPASS_IO(rowpass_dd, double, double)
 FLUPS_RZ(rz_d, double)
 
@@ -102,9 +104,18 @@ bool row_r2r_fits(const PassDesc& P, bool smooth) {
 }
 
 // columns: 5 and 7 on smooth (node-centred 129 x 161 x 97 165 -> 145, channel 160^3 184 -> 171); 3 stays
-// (channel 64 x 192 x 64 74 -> 77), powers of two too (channel 256^3 452 -> 483)
+// (channel 64 x 192 x 64 74 -> 77), powers of two too (channel 256^3 452 -> 483). Kinds I and IV of 7 times a power
+// of two, whose pre-maps pair values from both ends of the pencil, stay where smooth would run a radix of 14 (h = 112, 224,
+// 896, but for passes small enough for three stages): solves with h = 224, kind IV, 1024 pencils 12 % faster on smooth, 4096
+// and more 14-20 % slower, kind I 9-20 %; h = 896 3-8 %; h = 112 within 3 %
 bool col_r2r_fits(const PassDesc& P, bool smooth) {
-    return r2r_plan_fits(P, smooth, 3) && P.fa != P.d && P.src_s[P.fa] == 1 && P.dst_s[P.fa] == 1 && (P.n1 * P.n2) % P.na == 0;
+    int pf = 1, q = 0;
+    const int h = r2r_h(P.kind, P.n);
+    const bool k14 = P.kind == REDFT00 || P.kind == RODFT00 || P.kind == REDFT11 || P.kind == RODFT11;
+    if (!smooth && P.op == OP_R2R && split_pq(h, pf, q) && pf > 3 &&
+        !(pf == 7 && k14 && smooth_pen_wide(P, h)))
+        return false;
+    return r2r_plan_fits(P, smooth, 7) && P.fa != P.d && P.src_s[P.fa] == 1 && P.dst_s[P.fa] == 1 && (P.n1 * P.n2) % P.na == 0;
 }
 
 // pre / post twiddles of the row r2r kernels, (H + 1) complex each, exact to rounding

@@ -736,7 +736,9 @@ template <int PF, bool COL, typename TI, typename TO>
 void launch_pen_pf(int q, const PassDesc& P, hipStream_t s) {
     constexpr int H8 = PF * 8, H16 = PF * 16, H32 = PF * 32, H64 = PF * 64, H128 = PF * 128;
     switch (q) {
-        case 8: launch_pen_h<PF, 8, COL ? (H8 <= 64 ? 32 : 16) : 2048 / H8, COL, TI, TO>(P, s); break;
+        case 8:
+            if constexpr (!COL || PF == 3) launch_pen_h<PF, 8, COL ? (H8 <= 64 ? 32 : 16) : 2048 / H8, COL, TI, TO>(P, s);
+            break;
         case 16: launch_pen_h<PF, 16, COL ? (H16 <= 64 ? 32 : 16) : 2048 / H16, COL, TI, TO>(P, s); break;
         case 32: launch_pen_h<PF, 32, COL ? (H32 <= 64 ? 32 : H32 <= 256 ? 16 : 8) : 2048 / H32, COL, TI, TO>(P, s); break;
         case 64: launch_pen_h<PF, 64, COL ? (H64 <= 256 ? 16 : H64 <= 512 ? 8 : 4) : 2048 / H64, COL, TI, TO>(P, s); break;
@@ -1000,8 +1002,9 @@ void launch_col_r2r_t(const PassDesc& P, hipStream_t s) {
     int pf = 1, q = 0;
     split_pq(h, pf, q);
     if (pf != 1) {
-        FLUPS_REQUIRE(pf == 3, "column r2r: length %d", P.n);
-        launch_pen_pf<3, true, TI, TO>(q, P, s);
+        FLUPS_REQUIRE(pf == 3 || (pf == 7 && q >= 16), "column r2r: length %d", P.n);
+        if (pf == 3) launch_pen_pf<3, true, TI, TO>(q, P, s);
+        else launch_pen_pf<7, true, TI, TO>(q, P, s);   // kinds I and IV
         HIP_CHECK(hipGetLastError());
         return;
     }

@@ -422,6 +422,11 @@ static bool pen_plan(const PassDesc& P, int h, bool col, SmoothPlan& p) {
     if ((!col && h >= 224) || waves <= (q.rad[0] == 2 ? 512 : 1152)) p = q;
     return true;
 }
+// strided pencils for which the plan has a radix above 10
+bool smooth_pen_wide(const PassDesc& P, int h) {
+    SmoothPlan p;
+    return pen_plan(P, h, true, p) && p.wide;
+}
 
 bool smooth_col_tile(PassDesc& P, int n) {
     if (!smooth_plan(n, P.sm)) return false;
