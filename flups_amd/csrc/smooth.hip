@@ -408,10 +408,11 @@ bool smooth_plan(int M, SmoothPlan& p) { return smooth_plan_upto(M, 16, p, 2); }
 
 // Pencils: fewest stages, but three of radix 10 at most in the place of two where the two leave the chip short of waves: a stage
 // of radix R has M / R threads, so three stages have twice to four times the waves for one more trip through LDS. The
-// line lies at 1152 waves (256 CUs of four SIMDs), at 512 where the three begin with radix 2 (twice the threads of any
-// other stage). Measured on whole solves (FP64, two stages -> three) at 40 lengths from 20 to 256: up to 1024 waves
-// 0-30 % faster (32 x 320 x 32 walls in x and y, h = 160: 17-20 %), at 1152 from 5 % slower to 8 % faster, from 1500 up to
-// 20 % slower (h = 100); beginning with 2, up to 640 waves 1-20 % faster, at 1024 from 4 % slower to 7 % faster.
+// line lies at 1344 waves (five a CU), at 512 where the three begin with radix 2 (twice the threads of any other
+// stage). Measured on whole solves (FP64, two stages -> three) at 40 lengths from 20 to 256: up to 1024 waves
+// 0-30 % faster (32 x 320 x 32 walls in x and y, h = 160: 17-20 %), at 1152 to 1300 from 5 % slower (h = 63) to 10 % faster
+// (h = 80), from 1500 up to 20 % slower (h = 100); beginning with 2, up to 640 waves 1-20 % faster, at 1024 from 4 %
+// slower to 7 % faster.
 // Rows from 224 points on, whose two radices are both 14 or more, take three always (rows of 512 periodic points: 10-18 %
 // faster up to the largest fields; columns of that length 4 % slower to 14 % faster, left at the line).
 static bool pen_plan(const PassDesc& P, int h, bool col, SmoothPlan& p) {
@@ -419,7 +420,7 @@ static bool pen_plan(const PassDesc& P, int h, bool col, SmoothPlan& p) {
     SmoothPlan q;
     if (p.nst != 2 || !smooth_plan_upto(h, 10, q, 3)) return true;
     const long long waves = (long long)P.n1 * P.n2 * P.comps * p.T / 64;
-    if ((!col && h >= 224) || waves <= (q.rad[0] == 2 ? 512 : 1152)) p = q;
+    if ((!col && h >= 224) || waves <= (q.rad[0] == 2 ? 512 : 1344)) p = q;
     return true;
 }
 // strided pencils for which the plan has a radix above 10

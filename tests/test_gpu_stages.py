@@ -16,21 +16,21 @@ from tests.test_gpu_routes import launches
 pytestmark = pytest.mark.gpu
 
 E, O, P, U = 0, 1, 3, 4
-# (nglob, bc, center, lda): h = 80, 112, 160, 224, 225, 448, 896 columns of kinds I, II and IV in small fields, at 72 x 1024
+# (nglob, bc, center, lda): h = 80, 112, 160, 224, 225, 448, 896 columns of kinds I, II and IV in small fields, at 84 x 1024
 # threads of two stages and above; rows of 2 x 128, 225, 240 and 256 points; few columns times three components
 CASES = {
     "IV-160-few": ((64, 320, 16), [[E, E], [E, O], [P, P]], 1, 1),
-    "IV-160-limit": ((71, 320, 64), [[E, E], [O, E], [P, P]], 1, 1),   # 72 x 64 columns of 16 threads
-    "IV-160-many": ((72, 320, 64), [[E, E], [E, O], [P, P]], 1, 1),
+    "IV-160-limit": ((83, 320, 64), [[E, E], [O, E], [P, P]], 1, 1),   # 84 x 64 columns of 16 threads
+    "IV-160-many": ((84, 320, 64), [[E, E], [E, O], [P, P]], 1, 1),
     "IV-80-few": ((40, 160, 33), [[E, E], [E, O], [P, P]], 1, 1),
     "II-112-few": ((35, 224, 33), [[E, E], [O, O], [P, P]], 1, 1),
-    "II-112-many": ((70, 224, 75), [[E, E], [E, E], [P, P]], 1, 1),
-    "IV-112-many": ((70, 224, 75), [[E, E], [O, E], [P, P]], 1, 1),
-    "I-112-many": ((71, 113, 77), [[E, E], [O, O], [P, P]], 0, 1),
+    "II-112-many": ((70, 224, 90), [[E, E], [E, E], [P, P]], 1, 1),
+    "IV-112-many": ((70, 224, 90), [[E, E], [O, E], [P, P]], 1, 1),
+    "I-112-many": ((71, 113, 89), [[E, E], [O, O], [P, P]], 0, 1),
     "IV-224-few": ((33, 448, 32), [[E, E], [E, O], [P, P]], 1, 1),
-    "IV-224-many": ((72, 448, 65), [[E, E], [E, O], [P, P]], 1, 1),
-    "I-224-many": ((75, 225, 67), [[O, O], [E, E], [P, P]], 0, 1),
-    "semi-224": ((75, 113, 67), [[O, O], [E, U], [P, P]], 0, 1),
+    "IV-224-many": ((72, 448, 75), [[E, E], [E, O], [P, P]], 1, 1),
+    "I-224-many": ((75, 225, 75), [[O, O], [E, E], [P, P]], 0, 1),
+    "semi-224": ((75, 113, 75), [[O, O], [E, U], [P, P]], 0, 1),
     "I-896": ((33, 897, 33), [[O, O], [O, O], [P, P]], 0, 1),
     "IV-225": ((34, 450, 30), [[E, E], [O, E], [P, P]], 1, 1),
     "IV-448": ((33, 896, 32), [[E, E], [E, O], [P, P]], 1, 1),
