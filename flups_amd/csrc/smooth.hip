@@ -412,21 +412,21 @@ bool smooth_plan(int M, SmoothPlan& p) { return smooth_plan_upto(M, 16, p, 2); }
 // stage). Measured on whole solves (FP64, two stages -> three) at 40 lengths from 20 to 256: up to 1024 waves
 // 0-30 % faster (32 x 320 x 32 walls in x and y, h = 160: 17-20 %), at 1152 to 1300 from 5 % slower (h = 63) to 10 % faster
 // (h = 80), from 1500 up to 20 % slower (h = 100); beginning with 2, up to 640 waves 1-20 % faster, at 1024 from 4 %
-// slower to 7 % faster.
-// Rows from 224 points on, whose two radices are both 14 or more, take three always (rows of 512 periodic points: 10-18 %
-// faster up to the largest fields; columns of that length 4 % slower to 14 % faster, left at the line).
-static bool pen_plan(const PassDesc& P, int h, bool col, SmoothPlan& p) {
+// slower to 7 % faster. Powers of two keep two: their stages form some twiddles as products, and with one stage more
+// 256 x 128 x 96 open is 16-25 % further from the exact solution (all of its rows: Green's function of 512 points; the other
+// lengths: within 3 %, as often closer).
+static bool pen_plan(const PassDesc& P, int h, SmoothPlan& p) {
     if (!smooth_plan(h, p)) return false;
     SmoothPlan q;
-    if (p.nst != 2 || !smooth_plan_upto(h, 10, q, 3)) return true;
+    if (p.nst != 2 || (h & (h - 1)) == 0 || !smooth_plan_upto(h, 10, q, 3)) return true;
     const long long waves = (long long)P.n1 * P.n2 * P.comps * p.T / 64;
-    if ((!col && h >= 224) || waves <= (q.rad[0] == 2 ? 512 : 1344)) p = q;
+    if (waves <= (q.rad[0] == 2 ? 512 : 1344)) p = q;
     return true;
 }
 // strided pencils for which the plan has a radix above 10
 bool smooth_pen_wide(const PassDesc& P, int h) {
     SmoothPlan p;
-    return pen_plan(P, h, true, p) && p.wide;
+    return pen_plan(P, h, p) && p.wide;
 }
 
 bool smooth_col_tile(PassDesc& P, int n) {
@@ -442,7 +442,7 @@ void launch_smooth_col(const PassDesc& P, hipStream_t s) {
 // about 128 threads a block of contiguous pencils (64: 48, 128: 36, 256: 37, 512: 45 us a pass of 200 reals),
 // 16 neighbours of strided ones (128-byte rows; 4: 67, 8: 56, 16: 48, 32: 67 us a pass of 100 reals)
 bool smooth_pen_tile(PassDesc& P, int h, bool col) {
-    if (!pen_plan(P, h, col, P.sm)) return false;
+    if (!pen_plan(P, h, P.sm)) return false;
     if (col) {
         P.ppb = fit_tile(16, P.sm.T, [&](int np) { return pen_lds(P, true, np); });
         return P.ppb > 0;

@@ -1,5 +1,5 @@
-"""Stages of the mixed-radix pencil kernels by the size of the pass (three where two leave the chip short of waves, and from 224
-points on) and the thread-team columns of 7 times a power of two, on both sides of each rule, against the generic
+"""Stages of the mixed-radix pencil kernels by the size of the pass (three where two leave the chip short of waves, but
+for powers of two) and the thread-team columns of 7 times a power of two, on both sides of each rule, against the generic
 pass kernel: relative L2 and Linf <= 1e-12 (FP64), 1e-5 (FP32 storage)."""
 import numpy as np
 import pytest
